@@ -177,3 +177,33 @@ def test_few_rows_take_the_kept_halves(hip, N, K):
             assert torch.equal(ya.view(torch.int32), yb.view(torch.int32)), M
         else:
             assert rel_l2(_np(yb), _np(ya)) <= 2e-4, M
+
+
+@pytest.mark.parametrize("N,K,offset", [(4, 256, 0), (12, 768, 4), (68, 2304, 1)])
+def test_records_repack_and_halves_at_any_alignment(hip, N, K, offset):
+    """Source bytes and halves buffers off their 16- and 8-byte alignment, and
+    the rows written in two ranges: the same quants and halves as the
+    half-zero-point repack of the whole."""
+    import ctypes as C
+    from webgllm_amd import lib as L, ops
+    rng = np.random.default_rng(N + K + offset)
+    src = random_q4_k_bytes(rng, N, K, zero_scale_every=3, extreme=True)
+    buf = torch.zeros(src.size + 16, dtype=torch.uint8, device="cuda")
+    view = buf[offset:offset + src.size]
+    view.copy_(ops.to_device_bytes(src))
+    f16 = ops.Q4Matrix.from_q4_k(ops.to_device_bytes(src), N, K, native=False)
+    rec = ops.Q4Matrix(N, K, L.LAYOUT_ROWGROUP, L.ZERO_Q4K)
+    half = N // 8 * 4
+    row = K // 256 * 144
+    for r0, rows in ((0, half), (half, N - half)):
+        if rows:
+            rec.repack_q4_k(r0, rows, view[r0 * row:(r0 + rows) * row])
+    n = N * (K // 32)
+    out = torch.zeros(2 * n + 8, dtype=torch.int16, device="cuda")
+    o = offset % 2  # halves: 2-byte aligned at least
+    L.check(L.load().wg_q4k_record_halves(C.byref(rec.desc), out[o:].data_ptr(),
+                                          out[o + n:].data_ptr(), ops._stream()))
+    torch.cuda.synchronize()
+    assert torch.equal(rec.quants, f16.quants)
+    assert torch.equal(out[o:o + n], f16.scales.view(-1))
+    assert torch.equal(out[o + n:o + 2 * n], f16.zeros.view(-1))

@@ -122,69 +122,136 @@ __global__ void repack_q4_k_kernel(uint32_t *quants, uint16_t *scales, uint16_t 
 }
 
 // packQ4_K's quants with Q4_K's own scales kept (WG_ZERO_Q4K): thread =
-// (row group gi of the range, super-block s). The group's 4 rows' nibbles go
-// out as repack_q4_k_kernel writes them (15s for a constant block), and its
-// record gets the rows' d and dmin and the 8 blocks' 6-bit scales and mins.
-__global__ void repack_q4_k_rec_kernel(uint32_t *quants, uint8_t *recs, const uint8_t *src,
-                                       const int32_t *src_rows, int row0, int rows, int supers) {
-  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)(rows / 4) * supers) return;
-  const int gi = (int)(t / supers), s = (int)(t % supers);
-  const int g = row0 / 4 + gi, blocks = supers * 8;
-  uint8_t rec[Q4K_REC];
-  for (int k = 0; k < Q4K_REC; k++) rec[k] = 0;
-  uint4 *qv = reinterpret_cast<uint4 *>(quants);
+// (row group gi of the range, super-block s, block pair, row r of the group),
+// r fastest. Bound by memory: a thread loads its row's 16-byte header (one
+// line for the four pairs) and its pair's 32 nibble bytes and stores two
+// 16-byte block rows, as repack_q4_k_kernel writes them (15s for a constant
+// block); the record's 16 dwords come one from each of its 16 threads, the
+// 12-bit (scale, min) fields meeting by quad permutes. A thread a row group
+// and super-block, its bytes built in scratch, took 95 us on 28672 x 4096
+// (132 MB in and out); this takes 21.5 us (6.2 TB/s). A16: src is 16-byte aligned, so
+// every piece of a 144-byte super-block is.
+template <bool A16>
+__global__ __launch_bounds__(256) void repack_q4_k_rec_kernel(uint4 *quants, uint32_t *recs,
+                                                              const uint8_t *src,
+                                                              const int32_t *src_rows, int row0,
+                                                              uint32_t threads, int supers) {
+  // 32-bit thread counts: 2^32 threads would be a 155 GB matrix, which the
+  // device cannot hold beside its source (a 64-bit division cost more)
+  const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= threads) return;  // (threads: a multiple of 16, so whole records leave)
+  const int r = (int)(t & 3), pair = (int)(t >> 2) & 3;
+  const uint32_t gs = t >> 4;
+  const int gi = (int)(gs / (uint32_t)supers), s = (int)(gs % (uint32_t)supers);
+  const int i = 4 * gi + r;
+  const uint8_t *p = src + ((int64_t)(src_rows ? src_rows[i] : i) * supers + s) * 144;
+  auto piece = [&](int k) {
+    if constexpr (A16) return reinterpret_cast<const uint4 *>(p)[k];
+    const uint8_t *q = p + 16 * k;
+    return make_uint4(ld32_unaligned(q), ld32_unaligned(q + 4), ld32_unaligned(q + 8),
+                      ld32_unaligned(q + 12));
+  };
+  const uint4 hd = piece(0), a = piece(1 + 2 * pair), b = piece(2 + 2 * pair);
+  // the pair's two (scale, min) fields from the 12 scale bytes (hd.y, z, w),
+  // as q4k_scale_min decodes them
+  const int sh = 16 * (pair & 1);  // blocks 2 pair, 2 pair + 1: bytes sh / 8, sh / 8 + 1
+  uint32_t f[2];
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const uint32_t s0 = hd.y >> (sh + 8 * j), s4 = hd.z >> (sh + 8 * j),
+                   s8 = hd.w >> (sh + 8 * j);
+    f[j] = pair < 2 ? (s0 & 63u) | (s4 & 63u) << 6
+                    : ((s8 & 15u) | (s0 >> 2 & 0x30u)) | ((s8 >> 4 & 15u) | (s4 >> 2 & 0x30u)) << 6;
+  }
+  const double d = half_to_float((uint16_t)hd.x);
   const uint32_t LOW = 0x0f0f0f0fu;
-  for (int r = 0; r < 4; r++) {
-    const int i = 4 * gi + r;
-    const int sr = src_rows ? src_rows[i] : i;
-    const uint8_t *p = src + ((int64_t)sr * supers + s) * 144;
-    for (int k = 0; k < 4; k++) rec[4 * r + k] = p[k];
-    const double d = half_to_float(ld16_unaligned(p));
-    const double dmin = half_to_float(ld16_unaligned(p + 2));
-    for (int pair = 0; pair < 4; pair++) {
-      const uint8_t *at = p + 16 + pair * 32;
-      uint32_t lo[4], hi[4];
-      for (int w = 0; w < 4; w++) {
-        uint32_t a = ld32_unaligned(at + 4 * w), b = ld32_unaligned(at + 16 + 4 * w);
-        lo[w] = (a & LOW) | ((b & LOW) << 4);
-        hi[w] = ((a >> 4) & LOW) | (b & ~LOW);
-      }
-      for (int j2 = 0; j2 < 2; j2++) {
-        const int j = 2 * pair + j2;
-        int sc, mn;
-        q4k_scale_min(p + 4, j, &sc, &mn);
-        q4k_rec_put(rec, j, r, sc, mn);
-        uint16_t dq, zq;
-        const bool constant = q4k_block_dz(d, dmin, sc, mn, &dq, &zq);
-        const uint32_t *w = j2 ? hi : lo;
-        qv[((int64_t)g * blocks + s * 8 + j) * 4 + r] =
-            constant ? make_uint4(0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu)
-                     : make_uint4(w[0], w[1], w[2], w[3]);
-      }
-    }
+  const uint32_t av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
+  // 15s where d' = half(d sc) is zero (packQ4_K's constant block)
+  const uint32_t c0 = double_to_half_ref(d * (int)(f[0] & 63u)) & 0x7fffu ? 0u : ~0u;
+  const uint32_t c1 = double_to_half_ref(d * (int)(f[1] & 63u)) & 0x7fffu ? 0u : ~0u;
+  uint32_t lo[4], hi[4];
+#pragma unroll
+  for (int w = 0; w < 4; w++) {
+    lo[w] = (av[w] & LOW) | ((bv[w] & LOW) << 4) | c0;
+    hi[w] = ((av[w] >> 4) & LOW) | (bv[w] & ~LOW) | c1;
   }
-  uint4 *o = reinterpret_cast<uint4 *>(recs + ((int64_t)g * supers + s) * Q4K_REC);
-  for (int k = 0; k < Q4K_REC / 16; k++) {
-    uint32_t v[4];
-    for (int w = 0; w < 4; w++) v[w] = ld32_unaligned(rec + 16 * k + 4 * w);
-    o[k] = make_uint4(v[0], v[1], v[2], v[3]);
-  }
+  const int64_t gsd = (int64_t)(row0 / 4) * supers + gs;  // the record's index
+  uint4 *o = quants + gsd * 32 + pair * 8 + r;
+  o[0] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+  o[4] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+  // the pair's 96 bits from the quad's fields; lane 3 writes row `pair`'s d, dmin
+  const uint32_t ff = f[0] | f[1] << 16;
+  const int quad = (threadIdx.x & 63) & ~3;
+  uint32_t q[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) q[k] = __shfl(ff, quad + k, 64);
+  const uint32_t head = __shfl(hd.x, quad + pair, 64);
+  const uint32_t l[4] = {q[0] & 0xffffu, q[1] & 0xffffu, q[2] & 0xffffu, q[3] & 0xffffu};
+  const uint32_t h[4] = {q[0] >> 16, q[1] >> 16, q[2] >> 16, q[3] >> 16};
+  const uint32_t w0 = l[0] | l[1] << 12 | l[2] << 24;
+  const uint32_t w1 = l[2] >> 8 | l[3] << 4 | h[0] << 16 | h[1] << 28;
+  const uint32_t w2 = h[1] >> 4 | h[2] << 8 | h[3] << 20;
+  recs[gsd * (Q4K_REC / 4) + (r == 3 ? pair : 4 + 3 * pair + r)] =
+      r == 0 ? w0 : r == 1 ? w1 : r == 2 ? w2 : head;
 }
 
 // WG_ZERO_Q4K records -> packQ4_K's per-block (d', z') halves at the
-// WG_ZERO_F16 indices (the prefill GEMM's operands): thread = (row n, block b).
-__global__ void q4k_rec_expand_kernel(const uint8_t *recs, uint16_t *scales, uint16_t *zeros,
-                                      int N, int blocks) {
-  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)N * blocks) return;
-  const int n = (int)(t / blocks), b = (int)(t % blocks);
-  const uint8_t *rec = recs + ((int64_t)(n >> 2) * (blocks / 8) + b / 8) * Q4K_REC;
-  uint16_t dq, zq;
-  q4k_rec_dz(rec, b & 7, n & 3, &dq, &zq);
-  const int64_t si = ((int64_t)(n >> 2) * blocks + b) * 4 + (n & 3);
-  scales[si] = dq;
-  zeros[si] = zq;
+// WG_ZERO_F16 indices (the prefill GEMM's operands): thread = (row group,
+// block), its 4 rows' halves 8 bytes of each output. q4k_block_dz's values:
+// the quotient dmin m / d' of a 17-bit by an 11-bit significand is never
+// within 2^-36 of a float's rounding boundary without being on it, so the
+// float division (correctly rounded) gives the double quotient's float bit
+// for bit. 28672 x 4096: 21 us with a thread a row and block and the
+// division in doubles, 6.7 us now (22 MB). WIDE: the record is 16-byte
+// and the outputs are 8-byte aligned.
+template <bool WIDE>
+__global__ __launch_bounds__(256) void q4k_rec_expand_kernel(const uint8_t *recs,
+                                                             uint16_t *scales, uint16_t *zeros,
+                                                             uint32_t threads) {
+  const uint32_t t = blockIdx.x * 256 + threadIdx.x;  // group * blocks + block
+  if (t >= threads) return;
+  const int j = t & 7;  // (blocks a row: a multiple of 8)
+  const uint8_t *rec = recs + (int64_t)(t >> 3) * Q4K_REC;
+  auto word = [&](int at) {
+    if constexpr (WIDE) return *reinterpret_cast<const uint32_t *>(rec + at);
+    return ld32_unaligned(rec + at);
+  };
+  const int fw = 16 + 12 * (j >> 1) + 4 * (j & 1);
+  // the block's 48 bits: 4 rows' (scale, min)
+  const uint64_t f = (((uint64_t)word(fw + 4) << 32) | word(fw)) >> (16 * (j & 1));
+  const uint32_t hw[4] = {word(0), word(4), word(8), word(12)};
+  uint32_t dq[4], zq[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const uint32_t fr = (uint32_t)(f >> (12 * r));
+    const int sc = fr & 63, mn = fr >> 6 & 63;
+    // (hardware conversions: exact to float; float to half rounded to
+    // nearest even with subnormals, as double_to_half_ref)
+    const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)hw[r]);
+    const float dmin = (float)__builtin_bit_cast(_Float16, (uint16_t)(hw[r] >> 16));
+    const float scale = d * (float)sc, mins = dmin * (float)mn;  // exact
+    const _Float16 h = (_Float16)scale;
+    const float hv = (float)h;
+    if (hv != 0.0f && isfinite(hv) && isfinite(mins)) {
+      dq[r] = __builtin_bit_cast(uint16_t, h);
+      zq[r] = __builtin_bit_cast(uint16_t, (_Float16)(mins / hv));
+    } else {
+      uint16_t x, y;
+      q4k_block_dz(half_to_float((uint16_t)hw[r]), half_to_float((uint16_t)(hw[r] >> 16)), sc, mn,
+                   &x, &y);
+      dq[r] = x;
+      zq[r] = y;
+    }
+  }
+  if constexpr (WIDE) {
+    reinterpret_cast<uint2 *>(scales)[t] = make_uint2(dq[0] | dq[1] << 16, dq[2] | dq[3] << 16);
+    reinterpret_cast<uint2 *>(zeros)[t] = make_uint2(zq[0] | zq[1] << 16, zq[2] | zq[3] << 16);
+  } else {
+    for (int r = 0; r < 4; r++) {
+      scales[4 * (int64_t)t + r] = (uint16_t)dq[r];
+      zeros[4 * (int64_t)t + r] = (uint16_t)zq[r];
+    }
+  }
 }
 
 // Q4_K super-blocks regrouped by rows of 4 (record (g * supers + s) * 4 + r):
@@ -428,8 +495,11 @@ inline unsigned grid_for(int64_t threads, int per) { return (unsigned)((threads 
 
 int launch_q4k_expand(const wg_q4_matrix *w, uint16_t *scales, uint16_t *zeros, hipStream_t s) {
   const int blocks = w->K / 32;
-  q4k_rec_expand_kernel<<<grid_for((int64_t)w->N * blocks, 256), 256, 0, s>>>(
-      (const uint8_t *)w->scales, scales, zeros, w->N, blocks);
+  const int64_t n = (int64_t)(w->N / 4) * blocks;
+  const bool wide = ((uintptr_t)w->scales & 15) == 0 &&
+                    (((uintptr_t)scales | (uintptr_t)zeros) & 7) == 0;
+  auto kernel = wide ? q4k_rec_expand_kernel<true> : q4k_rec_expand_kernel<false>;
+  kernel<<<grid_for(n, 256), 256, 0, s>>>((const uint8_t *)w->scales, scales, zeros, (uint32_t)n);
   return launched("Q4_K record expansion");
 }
 
@@ -497,10 +567,12 @@ int wg_repack_q4_k(const wg_q4_matrix *m, int32_t row0, int32_t rows, const void
   if (m->zero == WG_ZERO_Q4K) {
     WG_REQUIRE(row0 % 4 == 0 && rows % 4 == 0,
                "wg_repack_q4_k: rows must start and end on a row group");
-    const int64_t n = (int64_t)(rows / 4) * supers;
-    repack_q4_k_rec_kernel<<<grid_for(n, 64), 64, 0, as_stream(stream)>>>(
-        (uint32_t *)m->quants, (uint8_t *)m->scales, (const uint8_t *)src, src_rows, row0, rows,
-        supers);
+    const int64_t n = (int64_t)(rows / 4) * supers * 16;
+    auto kernel = ((uintptr_t)src & 15) == 0 ? repack_q4_k_rec_kernel<true>
+                                             : repack_q4_k_rec_kernel<false>;
+    kernel<<<grid_for(n, 256), 256, 0, as_stream(stream)>>>(
+        (uint4 *)m->quants, (uint32_t *)m->scales, (const uint8_t *)src, src_rows, row0,
+        (uint32_t)n, supers);
     return launched("wg_repack_q4_k");
   }
   int64_t n = (int64_t)rows * supers * 4;

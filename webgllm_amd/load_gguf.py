@@ -209,14 +209,14 @@ class _Uploader:
         if types == {G.Q4_K} and K % 256 == 0:
             # packQ4_K's quants with Q4_K's own scales and mins kept (0.5625
             # bytes a weight; dequant rebuilds packQ4_K's halves bit for bit)
-            m = ops.Q4Matrix(N, K, L.LAYOUT_ROWGROUP, L.ZERO_Q4K, device=self.device)
+            m = ops.Q4Matrix(N, K, L.LAYOUT_ROWGROUP, L.ZERO_Q4K, device=self.device, fill=False)
             m.repack_q4_k(0, N, self._cat(parts), src_rows)
             m.prompt_desc()  # packQ4_K's halves for prompts and few-token batches
         elif G.Q4_0 in types:
             if types != {G.Q4_0}:
                 raise ValueError(f"GGUF: {parts[0][0]} can't be combined with "
                                  f"{', '.join(n for n, _ in parts[1:])}")
-            m = ops.Q4Matrix(N, K, L.LAYOUT_ROWGROUP, L.ZERO_8, device=self.device)
+            m = ops.Q4Matrix(N, K, L.LAYOUT_ROWGROUP, L.ZERO_8, device=self.device, fill=False)
             m.repack_q4_0(0, N, self._cat(parts), src_rows)
         else:
             bad = [n for (n, _), t in zip(parts, infos) if t.type not in _EIGHT_BIT]
@@ -224,7 +224,7 @@ class _Uploader:
                 raise ValueError(f"GGUF: {bad[0]} has tensor type {self.info(bad[0]).type}, "
                                  "which this loader doesn't take (Q4_0, Q8_0, Q4_1, Q4_K, "
                                  "Q5_K, Q6_K, F16, F32 do)")
-            m = ops.Q4Matrix(N, K, L.LAYOUT_Q8, L.ZERO_8, device=self.device)
+            m = ops.Q4Matrix(N, K, L.LAYOUT_Q8, L.ZERO_8, device=self.device, fill=False)
             if types == {G.Q8_0}:
                 m.repack_q8_0(0, N, self._cat(parts), src_rows)
             elif G.Q8_0 in types:

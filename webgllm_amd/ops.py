@@ -55,19 +55,24 @@ class Q4Matrix:
     header)."""
 
     def __init__(self, N: int, K: int, layout: int = L.LAYOUT_ROWGROUP, zero: int = L.ZERO_8,
-                 device="cuda"):
+                 device="cuda", fill: bool = True):
+        """fill=False leaves the arrays as allocated: for a caller whose
+        repack writes every row (a 28672 x 4096 Q4_K upload's zero fills
+        took 15 of 154 us)."""
         lib = L.load()
+        alloc = torch.zeros if fill else torch.empty
         qb, sb, zb = C.c_size_t(), C.c_size_t(), C.c_size_t()
         L.check(lib.wg_q4_sizes(N, K, layout, zero, C.byref(qb), C.byref(sb), C.byref(zb)))
         self.N, self.K, self.layout, self.zero = N, K, layout, zero
-        self.quants = torch.zeros(qb.value, dtype=torch.uint8, device=device)
-        self.scales = torch.zeros(max(sb.value, 2) // 2, dtype=torch.int16, device=device) \
+        self.quants = alloc(qb.value, dtype=torch.uint8, device=device)
+        self.scales = alloc(max(sb.value, 2) // 2, dtype=torch.int16, device=device) \
             if sb.value else None
         self.zeros = None
         if zb.value:
-            self.zeros = torch.full((zb.value,), 8, dtype=torch.uint8, device=device) \
-                if zero == L.ZERO_U8 else torch.zeros(zb.value // 2, dtype=torch.int16,
-                                                      device=device)
+            self.zeros = alloc(zb.value, dtype=torch.uint8, device=device) \
+                if zero == L.ZERO_U8 else alloc(zb.value // 2, dtype=torch.int16, device=device)
+            if fill and zero == L.ZERO_U8:
+                self.zeros.fill_(8)
         self.desc = L.Q4MatrixDesc(N, K, layout, zero, _p(self.quants), _p(self.scales),
                                    _p(self.zeros))
 
@@ -79,7 +84,7 @@ class Q4Matrix:
     # --- load-time repacking (the reference's loaders' packers, on the GPU)
     @classmethod
     def from_q4_0(cls, src: torch.Tensor, N: int, K: int, src_rows=None) -> "Q4Matrix":
-        m = cls(N, K, L.LAYOUT_ROWGROUP, L.ZERO_8, device=src.device)
+        m = cls(N, K, L.LAYOUT_ROWGROUP, L.ZERO_8, device=src.device, fill=False)
         m.repack_q4_0(0, N, src, src_rows)
         return m
 
@@ -90,18 +95,18 @@ class Q4Matrix:
         (native), packQ4_K's row groups with half zero points, or (records)
         the same quants with Q4_K's own scales kept (ZERO_Q4K)."""
         if native:
-            m = cls(N, K, L.LAYOUT_Q4K, L.ZERO_8, device=src.device)
+            m = cls(N, K, L.LAYOUT_Q4K, L.ZERO_8, device=src.device, fill=False)
             m.repack_q4_k_native(0, N, src, src_rows)
         else:
             m = cls(N, K, L.LAYOUT_ROWGROUP, L.ZERO_Q4K if records else L.ZERO_F16,
-                    device=src.device)
+                    device=src.device, fill=False)
             m.repack_q4_k(0, N, src, src_rows)
         return m
 
     @classmethod
     def from_q8_0(cls, src: torch.Tensor, N: int, K: int, src_rows=None) -> "Q4Matrix":
         """An 8-bit matrix from GGUF Q8_0 rows (packQ8_0)."""
-        m = cls(N, K, L.LAYOUT_Q8, L.ZERO_8, device=src.device)
+        m = cls(N, K, L.LAYOUT_Q8, L.ZERO_8, device=src.device, fill=False)
         m.repack_q8_0(0, N, src, src_rows)
         return m
 
@@ -109,14 +114,14 @@ class Q4Matrix:
     def from_floats_q8(cls, values: torch.Tensor) -> "Q4Matrix":
         """An 8-bit matrix quantized from float32 rows [N, K] (quantizeQ8)."""
         N, K = values.shape
-        m = cls(N, K, L.LAYOUT_Q8, L.ZERO_8, device=values.device)
+        m = cls(N, K, L.LAYOUT_Q8, L.ZERO_8, device=values.device, fill=False)
         m.quantize_q8(0, N, values)
         return m
 
     @classmethod
     def from_q6_k(cls, src: torch.Tensor, N: int, K: int, src_rows=None) -> "Q4Matrix":
         """A 6-bit matrix from GGUF Q6_K rows (packQ6_K)."""
-        m = cls(N, K, L.LAYOUT_Q6K, L.ZERO_8, device=src.device)
+        m = cls(N, K, L.LAYOUT_Q6K, L.ZERO_8, device=src.device, fill=False)
         m.repack_q6_k(0, N, src, src_rows)
         return m
 
@@ -124,7 +129,7 @@ class Q4Matrix:
     def from_nbits(cls, quant: torch.Tensor, scales: torch.Tensor, zp, N: int, K: int,
                    src_rows=None) -> "Q4Matrix":
         m = cls(N, K, L.LAYOUT_ROWGROUP, L.ZERO_U8 if zp is not None else L.ZERO_8,
-                device=quant.device)
+                device=quant.device, fill=False)
         m.repack_nbits(0, N, quant, scales, zp, src_rows)
         return m
 
