@@ -876,7 +876,7 @@ def workload_sample_pick(args):
                          f"repetitions ({spent:.1f} s)"}
     roof = {"bound": "hbm", "achieved": round(gbps, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
             "frac": round(gbps / HBM_PEAK_GBPS, 5), "traffic": None,
-            "kernel": "chunk_max_kernel + chunk_gather_kernel (one row, 128256 logits, 64 chunks)",
+            "kernel": "chunk_max_kernel + chunk_rank_gather_kernel (one row, 128256 logits, 64 chunks)",
             "bytes_per_launch": algo, "avg_launch_us": round(ms * 1e3, 2), "launches": reps}
     cfg = {"workload": "sampling pick of one 128256-logit row: penalties, best 64 chunks, "
                        "then the host sampler", "pick_and_sample_ms": round(host_ms, 3),

@@ -81,3 +81,21 @@ def test_sampling_from_candidates_equals_full_vocabulary(hip, settings):
     assert np.array_equal(d.p[o1], dfull.p[o2])
     for u in (0.0, 0.3, 0.77, 0.999):
         assert draw_at(d, u) == draw_at(dfull, u)
+
+
+@pytest.mark.parametrize("V,count", [(256, 1), (257, 2), (16384, 64), (16385, 64), (524288, 64)])
+def test_candidates_at_chunk_counts(hip, V, count):
+    """The fewest and the most chunks, a count of every chunk, and rows of
+    equal maxima and infinities, where only the order of indices ranks."""
+    from webgllm_amd import ops
+    rng = np.random.default_rng(V)
+    logits = rng.standard_normal((3, V)).astype(np.float32)
+    logits[1] = 2.0
+    logits[2] = -np.inf
+    logits[2, ::300] = np.inf
+    mask = rng.choice([0, 1, 2], V).astype(np.uint8)
+    want_c, want_v = O.pick_candidates(logits, count, mask=mask, penalty=1.1, presence=0.2)
+    got_c, got_v = ops.pick_candidates(_t(logits), count, mask=_t(mask), penalty=1.1,
+                                       presence_penalty=0.2)
+    assert np.array_equal(got_c.cpu().numpy(), want_c)
+    assert np.array_equal(got_v.cpu().numpy().view(np.uint32), want_v.view(np.uint32))
