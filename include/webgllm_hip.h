@@ -486,6 +486,16 @@ int wg_q4_gemm(const wg_q4_matrix *w, const uint16_t *A, int32_t M, int32_t lda,
                int32_t ldc, const float *residual, int32_t ldr, const float *row_scale,
                const int32_t *col_of, void *stream);
 
+/* C = A W^T for any number of rows and any N, for matrices too narrow for
+ * wg_q4_gemm (N not a multiple of 64: the b|a projection of a linear
+ * attention block): the products of wg_q4_gemv (exact, a block's scale
+ * applied to its float32 sum) on MFMA, so M rows give what a GEMV of each 8
+ * of them gives but for the order of the float32 sums. 8-bit matrices and
+ * 4-bit ones with integer zero points; others return WG_ERR_UNSUPPORTED
+ * before any launch. */
+int wg_q4_gemm_rows(const wg_q4_matrix *w, const uint16_t *A, int32_t M, int32_t lda, float *C,
+                    int32_t ldc, void *stream);
+
 /* The gate|up GEMM with the SwiGLU folded into it, for prompt batches (the
  * fused FFN passes of the reference's WebGPU kernels, src/gpu/native.ts:33,
  * and REDUCE_SWIGLU, kernels.ts:1066-1077): the matrix's rows come in

@@ -83,3 +83,27 @@ def test_block_matches_oracle(hip, D, H, dk, dv, rows):
         assert _rel(y.cpu().numpy(), want) < 1e-3, M
     assert _rel(blk.state.cpu().numpy(), ref.state) < 1e-3
     assert _rel(blk.conv_state[0].cpu().numpy()[:3], ref.conv) < 1e-5
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "nbits", "q8"])
+@pytest.mark.parametrize("N,K,M", [(4, 32, 1), (32, 2048, 9), (36, 96, 33), (68, 2080, 130)])
+def test_narrow_projection_of_many_rows(hip, fmt, N, K, M):
+    """gemm_rows: one block, an odd number of blocks, partial row and column
+    tiles, against the exact dequantized weights in float64 (products are
+    exact: float32 sums of K of them, 1e-6 relative)."""
+    from tests.test_gemm_gpu import _matrix
+    from webgllm_amd import ops
+    m = _matrix(fmt, N, K, seed=N + K)
+    rng = np.random.default_rng(M)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    y = ops.gemm_rows(m, torch.from_numpy(x).cuda()).cpu().numpy()
+    want = x.astype(np.float64) @ dense_of(m).astype(np.float64).T
+    assert _rel(y, want) < 1e-6
+
+
+def test_narrow_projection_declines_other_forms(hip):
+    from tests.test_gemm_gpu import _matrix
+    from webgllm_amd import ops
+    x = torch.zeros((9, 256), dtype=torch.float16, device="cuda")
+    for fmt in ("q4_k_rowgroup", "q4_k_records", "q6_k"):
+        assert ops.gemm_rows(_matrix(fmt, 8, 256, seed=1), x) is None

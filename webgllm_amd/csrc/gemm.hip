@@ -52,6 +52,7 @@
 
 #include "common.h"
 #include "dot.h"
+#include "gemm_core.h"
 #include "kernels.h"
 #include "lds_load.h"
 
@@ -107,10 +108,6 @@ __device__ inline void dequant8(uint2 bytes, uint16_t scale_bits, float zero, ha
     }
   }
 }
-
-// The weight form of a launch: the three zero-point kinds of 4-bit row
-// groups, or Q8 for WG_LAYOUT_Q8 (signed bytes, no zero point).
-constexpr int Q8 = 3;
 
 // 8 code bytes of one weight row for each K = 16 step of a block (weights
 // 8h.. and 16 + 8h..) -> the two operands as half(d q), rounded once:

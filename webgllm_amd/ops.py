@@ -266,6 +266,23 @@ def gemm(m: Q4Matrix, a16: torch.Tensor, out: torch.Tensor | None = None,
     return out
 
 
+def gemm_rows(m: Q4Matrix, a16: torch.Tensor):
+    """A W^T for M rows of a matrix too narrow for gemm (N not a multiple of
+    64), with gemv's exact products, in one launch. Returns None, having
+    launched nothing, for a matrix the kernel does not read."""
+    if a16.dtype not in (torch.float16, torch.int16):
+        raise ValueError("activations must be halves")
+    a16 = _dev(a16)
+    M = a16.shape[0]
+    out = torch.empty((M, m.N), dtype=torch.float32, device=a16.device)
+    rc = L.load().wg_q4_gemm_rows(C.byref(m.desc), _p(a16), M, a16.shape[1], _p(out), m.N,
+                                  _stream())
+    if rc == L.ERR_UNSUPPORTED:
+        return None
+    L.check(rc)
+    return out
+
+
 def gemm_swiglu(m: Q4Matrix, a16: torch.Tensor, out: torch.Tensor | None = None,
                 row_scale: torch.Tensor | None = None, kept: bool = True) -> torch.Tensor:
     """half(silu(gate) * up) [M, N / 2] of A W^T on MFMA, for a gate|up
