@@ -150,6 +150,33 @@ def test_delta_conv_matches_oracle(hip, M, C, W):
         assert np.array_equal(st_out.cpu().numpy()[:W - 1], want_state)
 
 
+@pytest.mark.parametrize("M", [8, 9, 15, 301])
+@pytest.mark.parametrize("C,W", [(4, 2), (1028, 3), (1024, 4)])
+def test_delta_conv_rows_equal_the_general_kernel(hip, M, C, W):
+    """Batches whose strides and arrays allow 16-byte loads run 8 rows a
+    thread: the outputs and states of the thread-an-output kernel (rows one
+    float further apart) bit for bit, the state from rows of the batch or,
+    where it is short, of the old state."""
+    from webgllm_amd import ops
+    rng = np.random.default_rng(M + C + W)
+    x = _t(rng.standard_normal((M, C + 4)).astype(np.float32))
+    odd = torch.zeros((M, C + 5), device="cuda")
+    odd[:, :C + 4] = x
+    taps = _t((rng.standard_normal((C, W)) * 0.5).astype(np.float32))
+    st = _t(rng.standard_normal((W - 1, C)).astype(np.float32))
+    s1, s2 = torch.empty_like(st), torch.empty_like(st)
+    got, want = ops.delta_conv(x, C, taps, st, s1), ops.delta_conv(odd, C, taps, st, s2)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and torch.equal(s1, s2)
+
+
+@pytest.mark.parametrize("H,dk,dv,M,save_at", [(2, 20, 17, 50, 0), (1, 36, 16, 79, 15),
+                                               (3, 112, 127, 193, 129), (1, 128, 33, 17, 16)])
+def test_delta_chunked_at_tile_edges(hip, H, dk, dv, M, save_at):
+    """Dims and chunk rows that end inside a 16 x 16 tile."""
+    test_delta_chunked_matches_oracle(hip, H, dk, dv, M, save_at)
+
+
 @pytest.mark.parametrize("M,H,dv", [(1, 16, 128), (9, 3, 80), (4, 2, 256), (2, 5, 7)])
 def test_delta_norm_matches_oracle(hip, M, H, dv):
     from webgllm_amd import ops

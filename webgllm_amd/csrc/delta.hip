@@ -201,6 +201,61 @@ __global__ __launch_bounds__(256) void delta_conv_kernel(const float *in, int ld
   }
 }
 
+// The same of prompt batches: a thread takes 4 channels of CONV_ROWS rows,
+// its window of rows loaded once into registers (11 16-byte loads for 8
+// outputs). Bound by memory: 1500 x 6144 (74 MB in and out) took 54 us with
+// a thread an output, 16 us now (4.6 TB/s). Channels and strides are multiples of 4,
+// the arrays 16-byte aligned.
+constexpr int CONV_ROWS = 8;
+
+template <int W>
+__global__ __launch_bounds__(256) void delta_conv_rows_kernel(const float *in, int ldi, int M,
+                                                              int C, const float *taps,
+                                                              const float *state,
+                                                              float *state_out, float *out,
+                                                              int ldo) {
+  const int c = 4 * (int)(blockIdx.x * 256 + threadIdx.x), m0 = (int)blockIdx.y * CONV_ROWS;
+  if (c >= C) return;
+  // row t of the stream: the state's rows come before row 0
+  auto row = [&](int t) {
+    return *reinterpret_cast<const float4 *>(t >= 0 ? in + (int64_t)t * ldi + c
+                                                    : state + (int64_t)(W - 1 + t) * C + c);
+  };
+  float4 x[CONV_ROWS + W - 1];
+#pragma unroll
+  for (int k = 0; k < CONV_ROWS + W - 1; k++)
+    x[k] = row(min(m0 - (W - 1) + k, M - 1));
+  float w[4][W];
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+#pragma unroll
+    for (int k = 0; k < W; k++) w[q][k] = taps[(int64_t)(c + q) * W + k];
+#pragma unroll
+  for (int r = 0; r < CONV_ROWS; r++) {
+    if (m0 + r >= M) break;
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < W; k++) {
+      const float4 v = x[r + k];
+      acc[0] = fmaf(w[0][k], v.x, acc[0]);
+      acc[1] = fmaf(w[1][k], v.y, acc[1]);
+      acc[2] = fmaf(w[2][k], v.z, acc[2]);
+      acc[3] = fmaf(w[3][k], v.w, acc[3]);
+    }
+    float4 o;
+    o.x = acc[0] / (1.0f + expf(-acc[0]));
+    o.y = acc[1] / (1.0f + expf(-acc[1]));
+    o.z = acc[2] / (1.0f + expf(-acc[2]));
+    o.w = acc[3] / (1.0f + expf(-acc[3]));
+    *reinterpret_cast<float4 *>(out + (int64_t)(m0 + r) * ldo + c) = o;
+  }
+  if (m0 + CONV_ROWS >= M) {  // the last rows' thread: the new state
+#pragma unroll
+    for (int i = 0; i < W - 1; i++)
+      *reinterpret_cast<float4 *>(state_out + (int64_t)i * C + c) = row(M - (W - 1) + i);
+  }
+}
+
 // LIN_NORM: a wave per (row, head), up to 4 values a lane.
 __global__ __launch_bounds__(256) void delta_norm_kernel(const float *o, int ldo, int M, int H,
                                                          int dv, const float *z, int ldz,
@@ -245,14 +300,26 @@ __global__ __launch_bounds__(256) void delta_norm_kernel(const float *o, int ldo
 // S <- e^{G_last} S + K~^T D. `delta_chunk_prep_kernel` does the first
 // part for every (head, chunk) at once; `delta_chunk_chain_kernel` the
 // state chain, a workgroup per (head, 16 state columns).
+//
+// Every product runs on v_mfma_f32_16x16x4_f32 (float32 operands and sums,
+// twice the vector units' rate). A 16 x 16 x 16 product is 4 of them, step j
+// contracting k = 4 c + j for the lane groups c = lane / 16: an A operand is
+// then 4 consecutive floats of a row (one 16-byte read), and a result's 4
+// registers (rows 4 c .. 4 c + 3 of column lane % 16) are the next product's
+// B operand as they stand. So the solve, P U and P W stay in a wave's
+// registers, and prep writes each matrix in the order the chain's lanes read
+// it: a fragment (16 x 16, 4 floats a lane) is 1 KB in one load.
 
 constexpr int CH = 64;        // rows a chunk
+constexpr int CT = CH / 16;   // its row tiles
 constexpr int CMAX = 128;     // key and value dims the chunked form takes
-constexpr int RS = CMAX + 4;  // LDS row stride (floats) of the row tiles
-constexpr int AS = CH + 4;    // LDS row stride of A (then T) and P
-constexpr int CBW = 16;       // state columns a chain workgroup
-constexpr size_t PREP_LDS = (3 * CH * RS + 2 * CH * AS + 3 * CH) * sizeof(float);
-constexpr size_t CHAIN_LDS = (CMAX * CBW + 3 * CH * RS + CH * CBW) * sizeof(float);
+constexpr int KTM = CMAX / 16;
+constexpr int RS = CMAX + 4;  // LDS row stride (floats) of the row tiles: rows 4 banks apart
+constexpr int AS = CH + 4;    // LDS row stride of A and P
+constexpr int TS = 20;        // LDS row stride of the inverted diagonal blocks
+constexpr int CW = 8;         // waves a workgroup
+constexpr size_t PREP_LDS = (2 * CH * RS + 2 * CH * AS + CH * TS + 4 * CH) * sizeof(float);
+typedef float f4v __attribute__((ext_vector_type(4)));
 
 struct ChunkArgs {
   const float *qkv;
@@ -261,7 +328,10 @@ struct ChunkArgs {
   int ldba;
   const float *A, *dt;
   int H, dk, dv, M, first, nch;
-  float *U, *W, *Oi, *Qp, *Kt, *eg;  // [H][nch][CH][dv or dk]; eg [H][nch]
+  // fragments (256 floats) a (head, chunk): U, Oi [dv tile][row tile] as
+  // results; -W, Q' [row tile][dk tile] and K~^T [dk tile][row tile] as A
+  // operands; eg [H][nch]
+  float *U, *W, *Oi, *Qp, *Kt, *eg;
   float *state, *snap;
   int save_at;
   float *out;
@@ -273,330 +343,328 @@ __device__ inline void chunk_rows(const ChunkArgs &a, int c, int &c0, int &n) {
   n = min(c == 0 ? a.first : CH, a.M - c0);
 }
 
-__device__ inline float dot4(float4 x, float4 y) {
-  return fmaf(x.x, y.x, fmaf(x.y, y.y, fmaf(x.z, y.z, x.w * y.w)));
+// c + (16 x 16 A) (16 x 16 B)
+__device__ __forceinline__ f4v mma16(f4v a, f4v b, f4v c) {
+#pragma unroll
+  for (int j = 0; j < 4; j++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], c, 0, 0, 0);
+  return c;
 }
 
-__global__ __launch_bounds__(256) void delta_chunk_prep_kernel(ChunkArgs a) {
+// Bound by MFMA: 1920 of them (15,360 clocks over 4 SIMDs) a workgroup. As
+// vector code (one wave a SIMD, T by a serial forward substitution of 64
+// rows) 1500 rows of 16 heads took 141 us; this takes 46 us.
+__global__ __launch_bounds__(64 * CW) void delta_chunk_prep_kernel(ChunkArgs a) {
   extern __shared__ __align__(16) float sm[];
-  float *sq = sm, *sk = sq + CH * RS, *sv = sk + CH * RS;  // q^, k^, v rows (0 past n, dims)
-  float *sA = sv + CH * RS, *sP = sA + CH * AS;             // A (then T) and P
-  float *sG = sP + CH * AS, *sB = sG + CH, *sE = sB + CH;  // G, beta, e^G
+  float *sq = sm, *sk = sq + CH * RS;            // q^, k^ rows (0 past n, dims); then Q', -W
+  float *sA = sk + CH * RS, *sP = sA + CH * AS;  // -A and P
+  float *sT = sP + CH * AS;                      // (I + A_ii)^-1 of the diagonal blocks
+  float *sG = sT + CH * TS, *sB = sG + CH, *sE = sB + CH, *sL = sE + CH;  // G, beta, e^G, e^(Gl-G)
   const int c = blockIdx.x, h = blockIdx.y, t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int ln = lane & 15, lg = lane >> 4;
   int c0, n;
   chunk_rows(a, c, c0, n);
   const int K = a.H * a.dk, dk = a.dk, dv = a.dv;
-  {  // every load issued before the first store: thread t takes column t % 128 of rows 2u + t / 128
+  const int KT = (dk + 15) / 16, VT = (dv + 15) / 16;
+  // every load issued before the first store: thread t takes column t % 128
+  // of rows 4 u + t / 128; a wave its 16 value columns
+  f4v x[CT];  // this wave's value columns: rows 16 i + 4 lg + e, column 16 wave + ln
+  {
     const int i = t & (CMAX - 1), r0 = t >> 7;
-    float rq[CH / 2], rk[CH / 2], rv[CH / 2];
+    float rq[CH / 4], rk[CH / 4];
 #pragma unroll
-    for (int u = 0; u < CH / 2; u++) {
-      const int r = 2 * u + r0;
+    for (int u = 0; u < CH / 4; u++) {
+      const int r = 4 * u + r0;
       const float *row = a.qkv + (int64_t)(c0 + r) * a.ldq;
-      const bool in = r < n;
-      rq[u] = in && i < dk ? row[h * dk + i] : 0.0f;
-      rk[u] = in && i < dk ? row[K + h * dk + i] : 0.0f;
-      rv[u] = in && i < dv ? row[2 * K + h * dv + i] : 0.0f;
+      const bool in = r < n && i < dk;
+      rq[u] = in ? row[h * dk + i] : 0.0f;
+      rk[u] = in ? row[K + h * dk + i] : 0.0f;
     }
+    const int vj = 16 * wave + ln;
 #pragma unroll
-    for (int u = 0; u < CH / 2; u++) {
-      const int r = 2 * u + r0;
-      sq[r * RS + i] = rq[u];
-      sk[r * RS + i] = rk[u];
-      sv[r * RS + i] = rv[u];
+    for (int i2 = 0; i2 < CT; i2++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int r = 16 * i2 + 4 * lg + e;
+        x[i2][e] = r < n && vj < dv ? a.qkv[(int64_t)(c0 + r) * a.ldq + 2 * K + h * dv + vj] : 0.0f;
+      }
+#pragma unroll
+    for (int u = 0; u < CH / 4; u++) {
+      sq[(4 * u + r0) * RS + i] = rq[u];
+      sk[(4 * u + r0) * RS + i] = rk[u];
     }
   }
   if (t < CH) {  // wave 0: the gates (LIN_GATES) and G by a shuffle scan (linCum)
     float beta = 0.0f, g = 0.0f;
     if (t < n) {
       const float *gb = a.ba + (int64_t)(c0 + t) * a.ldba;
-      const float x = gb[a.H + h] + a.dt[h];
+      const float y = gb[a.H + h] + a.dt[h];
       beta = 1.0f / (1.0f + expf(-gb[h]));
-      g = a.A[h] * (fmaxf(x, 0.0f) + log1pf(expf(-fabsf(x))));
+      g = a.A[h] * (fmaxf(y, 0.0f) + log1pf(expf(-fabsf(y))));
     }
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
       const float y = __shfl_up(g, off, 64);
       if (lane >= off) g += y;
     }
+    const float gl = __shfl(g, n - 1, 64);
     sB[t] = beta;
     sG[t] = g;
     sE[t] = expf(g);
+    sL[t] = expf(gl - g);
+    if (t == 0) a.eg[h * a.nch + c] = expf(gl);
   }
   lds_barrier();
-  {  // LIN_PREP: four threads a row
-    const int r = t >> 2, part = t & 3;
+  {  // LIN_PREP: eight threads a row
+    const int r = t >> 3, part = t & 7;
     float ssq = 0.0f, ssk = 0.0f;
-    for (int i = part; i < dk; i += 4) {
+    for (int i = part; i < dk; i += 8) {
       ssq = fmaf(sq[r * RS + i], sq[r * RS + i], ssq);
       ssk = fmaf(sk[r * RS + i], sk[r * RS + i], ssk);
     }
-    ssq = quad_sum(ssq);
-    ssk = quad_sum(ssk);
+#pragma unroll
+    for (int off = 1; off < 8; off <<= 1) {
+      ssq += __shfl_xor(ssq, off, 64);
+      ssk += __shfl_xor(ssk, off, 64);
+    }
     const float invq = 1.0f / sqrtf((float)dk) / sqrtf(ssq + 1e-6f);
     const float invk = 1.0f / sqrtf(ssk + 1e-6f);
-    for (int i = part; i < dk; i += 4) {
+    for (int i = part; i < dk; i += 8) {
       sq[r * RS + i] *= invq;
       sk[r * RS + i] *= invk;
     }
   }
   lds_barrier();
-  {  // linGram: a 4 x 4 block of (row, key) pairs a thread, lower triangle only
-    const int rb = t >> 4, sb = t & 15;
-    float kk[4][4] = {}, qk[4][4] = {};
-    if (sb <= rb) {
-      for (int i = 0; i < dk; i += 4) {
-        float4 kr[4], qr[4], ks[4];
+  // linGram: the lower triangle's 10 tiles of K^ K^T and of Q^ K^T
+  for (int job = wave; job < CT * (CT + 1); job += CW) {
+    const int pair = job >> 1, which = job & 1;
+    const int ti = pair < 1 ? 0 : pair < 3 ? 1 : pair < 6 ? 2 : 3;
+    const int tj = pair - ti * (ti + 1) / 2;
+    const float *ra = (which ? sq : sk) + (16 * ti + ln) * RS + 4 * lg;
+    const float *rb = sk + (16 * tj + ln) * RS + 4 * lg;
+    f4v g[4] = {};  // four chains of sums: shorter, and so closer to exact
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-          kr[u] = *reinterpret_cast<const float4 *>(&sk[(4 * rb + u) * RS + i]);
-          qr[u] = *reinterpret_cast<const float4 *>(&sq[(4 * rb + u) * RS + i]);
-          ks[u] = *reinterpret_cast<const float4 *>(&sk[(4 * sb + u) * RS + i]);
-        }
-#pragma unroll
-        for (int x = 0; x < 4; x++)
-#pragma unroll
-          for (int y = 0; y < 4; y++) {
-            kk[x][y] += dot4(kr[x], ks[y]);
-            qk[x][y] += dot4(qr[x], ks[y]);
-          }
-      }
+    for (int s = 0; s < KTM; s++) {
+      if (s >= KT) break;
+      g[s & 3] = mma16(*reinterpret_cast<const f4v *>(ra + 16 * s),
+                       *reinterpret_cast<const f4v *>(rb + 16 * s), g[s & 3]);
     }
+    const f4v dots = (g[0] + g[1]) + (g[2] + g[3]);
 #pragma unroll
-    for (int x = 0; x < 4; x++)
-#pragma unroll
-      for (int y = 0; y < 4; y++) {
-        const int r = 4 * rb + x, s = 4 * sb + y;
-        const bool ok = r < n && s <= r;
-        const float e = ok ? expf(sG[r] - sG[s]) : 0.0f;
-        sA[r * AS + s] = ok && s < r ? sB[r] * e * kk[x][y] : 0.0f;
-        sP[r * AS + s] = ok ? e * qk[x][y] : 0.0f;
-      }
-  }
-  const float gl = sG[n - 1];
-  const int64_t base = (int64_t)(h * a.nch + c) * CH;
-  for (int idx = t; idx < n * dk; idx += 256) {
-    const int r = idx / dk, i = idx % dk;
-    a.Kt[(base + r) * dk + i] = expf(gl - sG[r]) * sk[r * RS + i];
-  }
-  if (t == 0) a.eg[h * a.nch + c] = expf(gl);
-  lds_barrier();
-  if (t < 64) {  // linSolve: T = (I + A)^-1 by forward substitution, lane = column
-    float Tc[CH];
-#pragma unroll
-    for (int r = 0; r < CH; r++) {
-      float acc[4] = {lane == r ? 1.0f : 0.0f, 0.0f, 0.0f, 0.0f};  // 4 chains, not one
-#pragma unroll
-      for (int s = 0; s < r; s++) acc[s & 3] = fmaf(-sA[r * AS + s], Tc[s], acc[s & 3]);
-      Tc[r] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-    }
-#pragma unroll
-    for (int r = 0; r < CH; r++) sA[r * AS + lane] = Tc[r];
-  }
-  lds_barrier();
-  // linUW, then linQO: 4 rows x 8 columns (16 apart) a thread
-  const int rb = t >> 4, jb = t & 15;
-  const int smax = min(4 * rb + 3, n - 1);
-  float u[4][8] = {}, w[4][8] = {};
-#pragma unroll 2
-  for (int s = 0; s <= smax; s++) {
-    const float bs = sB[s], be = bs * sE[s];
-    float tr[4];
-#pragma unroll
-    for (int x = 0; x < 4; x++) tr[x] = sA[(4 * rb + x) * AS + s];
-#pragma unroll
-    for (int y = 0; y < 8; y++) {
-      const float vv = sv[s * RS + jb + 16 * y] * bs, kv = sk[s * RS + jb + 16 * y] * be;
-#pragma unroll
-      for (int x = 0; x < 4; x++) {
-        u[x][y] = fmaf(tr[x], vv, u[x][y]);
-        w[x][y] = fmaf(tr[x], kv, w[x][y]);
-      }
+    for (int e = 0; e < 4; e++) {
+      const int r = 16 * ti + 4 * lg + e, s = 16 * tj + ln;
+      const float d = dots[e];
+      const bool ok = r < n && s <= r;
+      const float ex = ok ? expf(sG[r] - sG[s]) : 0.0f;
+      if (which) sP[r * AS + s] = ok ? ex * d : 0.0f;
+      else sA[r * AS + s] = ok && s < r ? -(sB[r] * ex * d) : 0.0f;
     }
   }
-  lds_barrier();  // every read of v and k^ is done: U and W take their places
+  // K~^T as A operands: fragment (dk tile, row tile s), lane rows 16 s + 4 lg ..
+  const int64_t hc = (int64_t)h * a.nch + c;
+  if (wave < KT) {
 #pragma unroll
-  for (int x = 0; x < 4; x++) {
-    const int r = 4 * rb + x;
+    for (int s = 0; s < CT; s++) {
+      f4v v;
 #pragma unroll
-    for (int y = 0; y < 8; y++) {
-      const int j = jb + 16 * y;
-      sv[r * RS + j] = u[x][y];
-      sk[r * RS + j] = w[x][y];
-      if (r < n && j < dv) a.U[(base + r) * dv + j] = u[x][y];
-      if (r < n && j < dk) a.W[(base + r) * dk + j] = w[x][y];
+      for (int e = 0; e < 4; e++) {
+        const int r = 16 * s + 4 * lg + e;
+        v[e] = sL[r] * sk[r * RS + 16 * wave + ln];
+      }
+      *reinterpret_cast<f4v *>(a.Kt + ((hc * KT + wave) * CT + s) * 256 + 4 * lane) = v;
     }
   }
   lds_barrier();
-  float o[4][8] = {}, qp[4][8];
+  if (wave < CT && lane < 16) {  // linSolve: (I + A_ii)^-1, forward substitution, lane = column
+    const float *Ai = sA + 16 * wave * AS + 16 * wave;  // (holds -A)
+    float Tc[16];
 #pragma unroll
-  for (int x = 0; x < 4; x++)
+    for (int r = 0; r < 16; r++) {
+      float acc[2] = {lane == r ? 1.0f : 0.0f, 0.0f};
 #pragma unroll
-    for (int y = 0; y < 8; y++) qp[x][y] = sE[4 * rb + x] * sq[(4 * rb + x) * RS + jb + 16 * y];
-#pragma unroll 2
-  for (int s = 0; s <= smax; s++) {
-    float pr[4];
-#pragma unroll
-    for (int x = 0; x < 4; x++) pr[x] = sP[(4 * rb + x) * AS + s];
-#pragma unroll
-    for (int y = 0; y < 8; y++) {
-      const float us = sv[s * RS + jb + 16 * y], ws = sk[s * RS + jb + 16 * y];
-#pragma unroll
-      for (int x = 0; x < 4; x++) {
-        o[x][y] = fmaf(pr[x], us, o[x][y]);
-        qp[x][y] = fmaf(-pr[x], ws, qp[x][y]);
-      }
+      for (int s = 0; s < r; s++) acc[s & 1] = fmaf(Ai[r * AS + s], Tc[s], acc[s & 1]);
+      Tc[r] = acc[0] + acc[1];
     }
+#pragma unroll
+    for (int r = 0; r < 16; r++) sT[(16 * wave + r) * TS + lane] = Tc[r];
+  }
+  lds_barrier();
+  // linUW by blocks: X_i = T_ii (R_i - sum_j<i A_ij X_j), this wave's value
+  // columns (R = beta V) and key columns (R = beta e^G K^).
+  const f4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f4v y[CT], qp[CT];
+#pragma unroll
+  for (int i = 0; i < CT; i++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int r = 16 * i + 4 * lg + e;
+      const float b = sB[r], ex = sE[r];
+      x[i][e] *= b;
+      y[i][e] = sk[r * RS + 16 * wave + ln] * (b * ex);
+      qp[i][e] = sq[r * RS + 16 * wave + ln] * ex;
+    }
+#pragma unroll
+  for (int i = 0; i < CT; i++) {
+#pragma unroll
+    for (int j = 0; j < i; j++) {  // (each block's sum by itself, then added)
+      const f4v m = *reinterpret_cast<const f4v *>(sA + (16 * i + ln) * AS + 16 * j + 4 * lg);
+      x[i] += mma16(m, x[j], zero);
+      y[i] += mma16(m, y[j], zero);
+    }
+    const f4v m = *reinterpret_cast<const f4v *>(sT + (16 * i + ln) * TS + 4 * lg);
+    x[i] = mma16(m, x[i], zero);
+    y[i] = mma16(m, y[i], zero);
   }
 #pragma unroll
-  for (int x = 0; x < 4; x++) {
-    const int r = 4 * rb + x;
-    if (r >= n) continue;
+  for (int i = 0; i < CT; i++) y[i] = -y[i];
+  // linQO: Oi = P U, Q' = e^G Q^ + P (-W)
+  f4v o[CT];
 #pragma unroll
-    for (int y = 0; y < 8; y++) {
-      const int j = jb + 16 * y;
-      if (j < dv) a.Oi[(base + r) * dv + j] = o[x][y];
-      if (j < dk) a.Qp[(base + r) * dk + j] = qp[x][y];
+  for (int i = 0; i < CT; i++) {
+    o[i] = zero;
+#pragma unroll
+    for (int j = 0; j <= i; j++) {
+      const f4v m = *reinterpret_cast<const f4v *>(sP + (16 * i + ln) * AS + 16 * j + 4 * lg);
+      o[i] += mma16(m, x[j], zero);
+      qp[i] += mma16(m, y[j], zero);
+    }
+  }
+  if (wave < VT) {
+#pragma unroll
+    for (int i = 0; i < CT; i++) {
+      const int64_t at = ((hc * VT + wave) * CT + i) * 256 + 4 * lane;
+      *reinterpret_cast<f4v *>(a.U + at) = x[i];
+      *reinterpret_cast<f4v *>(a.Oi + at) = o[i];
+    }
+  }
+  lds_barrier();  // every read of q^ and k^ is done: Q' and -W take their places
+#pragma unroll
+  for (int i = 0; i < CT; i++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int at = (16 * i + 4 * lg + e) * RS + 16 * wave + ln;
+      sk[at] = y[i][e];
+      sq[at] = qp[i][e];
+    }
+  lds_barrier();
+  if (wave < KT) {
+#pragma unroll
+    for (int i = 0; i < CT; i++) {
+      const int from = (16 * i + ln) * RS + 16 * wave + 4 * lg;
+      const int64_t at = ((hc * CT + i) * KT + wave) * 256 + 4 * lane;
+      *reinterpret_cast<f4v *>(a.W + at) = *reinterpret_cast<const f4v *>(sk + from);
+      *reinterpret_cast<f4v *>(a.Qp + at) = *reinterpret_cast<const f4v *>(sq + from);
     }
   }
 }
 
-constexpr int CT = 512;                   // chain threads
-constexpr int CG = CT / CBW;              // their groups (32)
-constexpr int DROWS = CH / CG;            // D and O rows a thread
-constexpr int SROWS = CMAX / CG;          // state rows a thread
-constexpr int SPT = CH * CMAX / 4 / CT;   // float4 of each staged tile a thread
+// A chunk's fragments for one chain wave: its row tile of -W and U (waves 0
+// to 3) or of Q' and Oi (4 to 7), its dk tile of K~^T, the decay.
+struct ChainIn {
+  f4v a[KTM], k[CT], u;
+  float e;
+};
 
-__device__ __forceinline__ void chain_fetch(const ChunkArgs &a, int c, int h, int t, int g,
-                                            int jj, bool col, float4 (&pw)[SPT],
-                                            float4 (&pq)[SPT], float4 (&pk)[SPT],
-                                            float (&pu)[DROWS], float (&po)[DROWS],
-                                            float &pe) {
-  int c0, n;
-  chunk_rows(a, c, c0, n);
-  const int64_t base = (int64_t)(h * a.nch + c) * CH;
-  const int dk = a.dk, dv = a.dv;
-#pragma unroll
-  for (int u = 0; u < SPT; u++) {
-    const int idx = t + CT * u, r = idx / (CMAX / 4), i = (idx % (CMAX / 4)) * 4;
-    pw[u] = pq[u] = pk[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (r < n && i < dk) {  // (a select of the two would put the zero in memory)
-      pw[u] = *reinterpret_cast<const float4 *>(&a.W[(base + r) * dk + i]);
-      pq[u] = *reinterpret_cast<const float4 *>(&a.Qp[(base + r) * dk + i]);
-      pk[u] = *reinterpret_cast<const float4 *>(&a.Kt[(base + r) * dk + i]);
-    }
-  }
-#pragma unroll
-  for (int x = 0; x < DROWS; x++) {
-    const int r = DROWS * g + x;
-    const bool in = r < n && col;
-    pu[x] = in ? a.U[(base + r) * dv + jj] : 0.0f;
-    po[x] = in ? a.Oi[(base + r) * dv + jj] : 0.0f;
-  }
-  pe = a.eg[h * a.nch + c];
-}
-
-__global__ __launch_bounds__(CT) void delta_chunk_chain_kernel(ChunkArgs a) {
-  extern __shared__ __align__(16) float sm[];
-  float *sS = sm;                                           // [CMAX][CBW] state block
-  float *sW = sS + CMAX * CBW, *sQ = sW + CH * RS, *sK = sQ + CH * RS;  // [CH][RS]
-  float *sD = sK + CH * RS;                                 // [CH][CBW]
+// A workgroup per (head, 16 state columns): waves 0 to 3 a row tile of D
+// each, 4 to 7 one of O, then every wave its 16 state rows. The state and D
+// pass between the waves through LDS as fragments. Bound by MFMA (384 a
+// chunk, 3072 clocks over 4 SIMDs) and the two exchanges a chunk. The
+// fragments come one chunk ahead. As vector code over LDS tiles a chunk took
+// 7.6 us, 1500 rows 184 us; this takes 66 us.
+__global__ __launch_bounds__(64 * CW) void delta_chunk_chain_kernel(ChunkArgs a) {
+  __shared__ __align__(16) float sS[2][KTM][256], sD[CT][256];
   // blockIdx.x is the head: the workgroups of one head (consecutive in
   // blockIdx.y, H apart in launch order) land on one XCD, whose L2 then
-  // serves the head's tiles to all of them.
-  const int h = blockIdx.x, t = threadIdx.x, j = t & (CBW - 1), g = t / CBW;
-  const int jj = blockIdx.y * CBW + j;
-  const bool col = jj < a.dv;
-  const int dk = a.dk, dv = a.dv;
-  float *Sh = a.state + (int64_t)h * dk * dv;
-  for (int i = g; i < CMAX; i += CG) sS[i * CBW + j] = col && i < dk ? Sh[(int64_t)i * dv + jj] : 0.0f;
-  // A chunk's W, Q', K~ tiles and this thread's U and Oi, fetched into
-  // registers one chunk ahead.
-  float4 pw[SPT], pq[SPT], pk[SPT];
-  float pu[DROWS], po[DROWS], pe;
-  chain_fetch(a, 0, h, t, g, jj, col, pw, pq, pk, pu, po, pe);
-  for (int c = 0; c < a.nch; c++) {
+  // serves the head's fragments to all of them.
+  const int h = blockIdx.x, vt = blockIdx.y, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ln = lane & 15, lg = lane >> 4, jj = 16 * vt + ln;
+  const int dk = a.dk, dv = a.dv, KT = (dk + 15) / 16, VT = (dv + 15) / 16;
+  const bool col = jj < dv, low = wave < CT;
+  const int tile = low ? wave : wave - CT;
+  float *Sh = a.state + (int64_t)h * dk * dv + jj;
+  f4v S;  // state rows 16 wave + 4 lg + e, column jj
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const int i = 16 * wave + 4 * lg + e;
+    S[e] = col && i < dk ? Sh[(int64_t)i * dv] : 0.0f;
+  }
+  *reinterpret_cast<f4v *>(&sS[0][wave][4 * lane]) = S;
+  const float *A0 = low ? a.W : a.Qp, *U0 = low ? a.U : a.Oi;
+  auto fetch = [&](ChainIn &f, int c) {
+    const int64_t hc = (int64_t)h * a.nch + c;
+    const float *pa = A0 + (hc * CT + tile) * KT * 256 + 4 * lane;
+    const float *pk = a.Kt + (hc * KT + min(wave, KT - 1)) * CT * 256 + 4 * lane;
+#pragma unroll
+    for (int s = 0; s < KTM; s++)  // (tiles past dk: the last again, unused)
+      f.a[s] = *reinterpret_cast<const f4v *>(pa + min(s, KT - 1) * 256);
+    f.u = *reinterpret_cast<const f4v *>(U0 + ((hc * VT + vt) * CT + tile) * 256 + 4 * lane);
+#pragma unroll
+    for (int s = 0; s < CT; s++) f.k[s] = *reinterpret_cast<const f4v *>(pk + s * 256);
+    f.e = a.eg[hc];
+  };
+  auto chunk = [&](const ChainIn &f, ChainIn &next, int c) {
     int c0, n;
     chunk_rows(a, c, c0, n);
+    const int p = c & 1;
+    fetch(next, min(c + 1, a.nch - 1));  // in flight while this chunk computes
+    // linChunkOut: D = U - W S, O = Oi + Q' S
+    f4v g[4] = {};  // four chains of sums: shorter, and so closer to exact
 #pragma unroll
-    for (int u = 0; u < SPT; u++) {
-      const int idx = t + CT * u, r = idx / (CMAX / 4), i = (idx % (CMAX / 4)) * 4;
-      *reinterpret_cast<float4 *>(&sW[r * RS + i]) = pw[u];
-      *reinterpret_cast<float4 *>(&sQ[r * RS + i]) = pq[u];
-      *reinterpret_cast<float4 *>(&sK[r * RS + i]) = pk[u];
+    for (int s = 0; s < KTM; s++) {
+      if (s >= KT) break;
+      const f4v b = *reinterpret_cast<const f4v *>(&sS[p][s][4 * lane]);
+      g[s & 3] = mma16(f.a[s], b, g[s & 3]);
     }
-    float d[DROWS], o[DROWS];
-#pragma unroll
-    for (int x = 0; x < DROWS; x++) {
-      d[x] = pu[x];
-      o[x] = po[x];
-    }
-    const float e = pe;
+    const f4v r0 = f.u + ((g[0] + g[1]) + (g[2] + g[3]));
+    if (low) *reinterpret_cast<f4v *>(&sD[tile][4 * lane]) = r0;
     lds_barrier();
-    if (c + 1 < a.nch)  // in flight while this chunk computes
-      chain_fetch(a, c + 1, h, t, g, jj, col, pw, pq, pk, pu, po, pe);
-    // linChunkOut: D = U - W S, O = Oi + Q' S, rows DROWS g ..
-    for (int i = 0; i < dk; i += 8) {  // dk is a multiple of 4: the operands of two steps first
-      float sv[8];
-      float4 wv[2][DROWS], qv[2][DROWS];
+    // linChunkState: S <- e^{G_last} S + K~^T D
+    f4v u[2] = {};
 #pragma unroll
-      for (int q = 0; q < 8; q++) sv[q] = sS[(i + q) * CBW + j];  // rows dk.. (< 128) are 0
+    for (int s = 0; s < CT; s++)
+      u[s & 1] = mma16(f.k[s], *reinterpret_cast<const f4v *>(&sD[s][4 * lane]), u[s & 1]);
 #pragma unroll
-      for (int q = 0; q < 2; q++)
+    for (int e = 0; e < 4; e++) S[e] = fmaf(f.e, S[e], u[0][e] + u[1][e]);
+    if (wave >= KT) S = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+    *reinterpret_cast<f4v *>(&sS[p ^ 1][wave][4 * lane]) = S;
+    if (!low && col) {
 #pragma unroll
-        for (int x = 0; x < DROWS; x++) {
-          wv[q][x] = *reinterpret_cast<const float4 *>(&sW[(DROWS * g + x) * RS + i + 4 * q]);
-          qv[q][x] = *reinterpret_cast<const float4 *>(&sQ[(DROWS * g + x) * RS + i + 4 * q]);
-        }
-#pragma unroll
-      for (int q = 0; q < 2; q++) {
-        const float4 s4 = make_float4(sv[4 * q], sv[4 * q + 1], sv[4 * q + 2], sv[4 * q + 3]);
-#pragma unroll
-        for (int x = 0; x < DROWS; x++) {
-          d[x] -= dot4(wv[q][x], s4);
-          o[x] += dot4(qv[q][x], s4);
-        }
+      for (int e = 0; e < 4; e++) {
+        const int r = 16 * tile + 4 * lg + e;
+        if (r < n) a.out[(int64_t)(c0 + r) * a.ldo + h * dv + jj] = r0[e];
       }
     }
+    if (a.snap && c0 + n == a.save_at && col) {
 #pragma unroll
-    for (int x = 0; x < DROWS; x++) {
-      const int r = DROWS * g + x;
-      sD[r * CBW + j] = r < n ? d[x] : 0.0f;
-      if (r < n && col) a.out[(int64_t)(c0 + r) * a.ldo + h * dv + jj] = o[x];
-    }
-    lds_barrier();
-    // linChunkState: S <- e^{G_last} S + K~^T D, state rows g + CG u
-    float acc[SROWS];
-#pragma unroll
-    for (int u = 0; u < SROWS; u++) acc[u] = e * sS[(g + CG * u) * CBW + j];
-    for (int r = 0; r < n; r += 4) {  // rows past n hold D = 0 and K~ = 0
-      float dr[4], kv[4][SROWS];
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        dr[q] = sD[(r + q) * CBW + j];
-#pragma unroll
-        for (int u = 0; u < SROWS; u++) kv[q][u] = sK[(r + q) * RS + g + CG * u];
+      for (int e = 0; e < 4; e++) {
+        const int i = 16 * wave + 4 * lg + e;
+        if (i < dk) a.snap[(int64_t)h * dk * dv + (int64_t)i * dv + jj] = S[e];
       }
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-#pragma unroll
-        for (int u = 0; u < SROWS; u++) acc[u] = fmaf(kv[q][u], dr[q], acc[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < SROWS; u++) {
-      const int i = g + CG * u;
-      sS[i * CBW + j] = acc[u];
-      if (a.snap && c0 + n == a.save_at && col && i < dk)
-        a.snap[(int64_t)h * dk * dv + (int64_t)i * dv + jj] = acc[u];
     }
     lds_barrier();
+  };
+  ChainIn f0, f1;
+  fetch(f0, 0);
+  lds_barrier();
+  for (int c = 0; c < a.nch; c += 2) {
+    chunk(f0, f1, c);
+    if (c + 1 < a.nch) chunk(f1, f0, c + 1);
   }
-  if (col)
-    for (int i = g; i < dk; i += CG) Sh[(int64_t)i * dv + jj] = sS[i * CBW + j];
+  if (col) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int i = 16 * wave + 4 * lg + e;
+      if (i < dk) Sh[(int64_t)i * dv] = S[e];
+    }
+  }
 }
 
 // Chunks of a batch of M rows whose first chunk has `first` rows.
 inline int chunk_count(int M, int first) { return M <= first ? 1 : 1 + (M - first + CH - 1) / CH; }
+
+// A chunk's fragments of `dim` columns, in floats.
+inline size_t fragment_floats(int dim) { return (size_t)((dim + 15) / 16) * CT * 256; }
 
 // The first chunk's rows: shorter, so that a chunk ends at save_at
 // (Engine.recurrenceChunks' rule), else CH.
@@ -639,9 +707,9 @@ int wg_delta_rule(const float *qkv, int32_t M, int32_t ldq, const float *ba, int
 size_t wg_delta_chunk_scratch_bytes(int32_t M, const wg_delta_shape *shape, int32_t save_at) {
   if (!shape || M < 1) return 0;
   const size_t nch = (size_t)chunk_count(M, first_rows(save_at));
-  return sizeof(float) * ((size_t)shape->heads * nch * CH *
-                              (2 * (size_t)shape->value_dim + 3 * (size_t)shape->key_dim) +
-                          (size_t)shape->heads * nch);
+  return sizeof(float) * (shape->heads * nch * (fragment_floats(shape->value_dim) * 2 +
+                                                fragment_floats(shape->key_dim) * 3) +
+                          shape->heads * nch);
 }
 
 int wg_delta_rule_chunked(const float *qkv, int32_t M, int32_t ldq, const float *ba,
@@ -667,20 +735,18 @@ int wg_delta_rule_chunked(const float *qkv, int32_t M, int32_t ldq, const float 
              scratch_bytes, need);
   WG_REQUIRE(((uintptr_t)scratch & 15) == 0, "wg_delta_rule_chunked: scratch not 16-byte aligned");
   int rc = raise_lds((const void *)delta_chunk_prep_kernel, (int)PREP_LDS);
-  if (!rc) rc = raise_lds((const void *)delta_chunk_chain_kernel, (int)CHAIN_LDS);
   if (rc) return rc;
   const int first = first_rows(save_at), nch = chunk_count(M, first);
-  const size_t rows = (size_t)H * nch * CH;
+  const size_t fv = (size_t)H * nch * fragment_floats(dv), fk = (size_t)H * nch * fragment_floats(dk);
   float *f = static_cast<float *>(scratch);
   ChunkArgs a{qkv, ldq, ba, ldba, A, dt_bias, H, dk, dv, M, first, nch,
-              f, f + rows * dv, f + rows * (dv + dk), f + rows * (2 * dv + dk),
-              f + rows * (2 * dv + 2 * dk), f + rows * (2 * dv + 3 * dk),
+              f, f + 2 * fv, f + fv, f + 2 * fv + fk, f + 2 * fv + 2 * fk, f + 2 * fv + 3 * fk,
               state, snapshot, save_at, out, ldo};
   hipStream_t s = as_stream(stream);
-  delta_chunk_prep_kernel<<<dim3(nch, H), 256, PREP_LDS, s>>>(a);
+  delta_chunk_prep_kernel<<<dim3(nch, H), 64 * CW, PREP_LDS, s>>>(a);
   rc = launched("wg_delta_rule_chunked");
   if (rc) return rc;
-  delta_chunk_chain_kernel<<<dim3(H, (dv + CBW - 1) / CBW), CT, CHAIN_LDS, s>>>(a);
+  delta_chunk_chain_kernel<<<dim3(H, (dv + 15) / 16), 64 * CW, 0, s>>>(a);
   return launched("wg_delta_rule_chunked");
 }
 
@@ -693,6 +759,15 @@ int wg_delta_conv(const float *in, int32_t M, int32_t ldi, int32_t C, int32_t W,
   const size_t sb = (size_t)(W - 1) * C * sizeof(float);
   WG_REQUIRE(W == 1 || (state && state_out && !overlaps(state, sb, state_out, sb)),
              "wg_delta_conv: %d taps need a state and a separate state_out", W);
+  const uintptr_t ptrs = (uintptr_t)in | (uintptr_t)out | (uintptr_t)state | (uintptr_t)state_out;
+  if (M >= CONV_ROWS && W >= 2 && W <= 4 && C % 4 == 0 && ldi % 4 == 0 && ldo % 4 == 0 &&
+      (ptrs & 15) == 0 && (M + CONV_ROWS - 1) / CONV_ROWS <= 65535) {
+    auto kernel = W == 2 ? delta_conv_rows_kernel<2>
+                         : W == 3 ? delta_conv_rows_kernel<3> : delta_conv_rows_kernel<4>;
+    kernel<<<dim3((C / 4 + 255) / 256, (M + CONV_ROWS - 1) / CONV_ROWS), 256, 0,
+             as_stream(stream)>>>(in, ldi, M, C, taps, state, state_out, out, ldo);
+    return launched("wg_delta_conv");
+  }
   const int64_t n = (int64_t)(M + W - 1) * C;
   delta_conv_kernel<<<(unsigned)((n + 255) / 256), 256, 0, as_stream(stream)>>>(
       in, ldi, M, C, W, taps, state, state_out, out, ldo);
