@@ -386,6 +386,26 @@ def test_attn_prefill_matches_decode_rows(hip, prefill_kernel):
         assert rel_l2(got[m], one[0]) <= 1e-4
 
 
+@pytest.mark.parametrize("waves", [1, 2, 3])
+@pytest.mark.parametrize("H,KV,hd", [(14, 2, 64), (32, 8, 128), (64, 2, 64)])
+@pytest.mark.parametrize("M,pos0", [(1, 0), (9, 22), (17, 47), (33, 63), (70, 190)])
+def test_attn_prefill_wave_splits(hip, waves, H, KV, hd, M, pos0):
+    """Each split of a workgroup's waves between queries and keys, every row:
+    fewer key steps than wave groups (one that had no key merges nothing),
+    last keys on and beside a step's edge, a last workgroup short of rows, 32
+    query heads a KV head."""
+    from webgllm_amd import lib as L
+    old = L.tuning_get("attn_prefill_mfma")
+    L.tuning_set("attn_prefill_mfma", waves)
+    try:
+        q, k, v, got = _prefill_case(H, KV, hd, M, pos0, seed=M + pos0, nan_past=True)
+    finally:
+        L.tuning_set("attn_prefill_mfma", old)
+    for m in range(M):
+        want = O.attention_f64(q[m], k, v, H, KV, hd, pos0 + m + 1, KV * hd)
+        assert rel_l2(got[m], want) <= 1e-3, m
+
+
 @pytest.mark.parametrize("M,D,W", [(1, 2048, 3), (5, 2048, 3), (8, 1024, 4), (40, 512, 3)])
 def test_short_conv_and_accept(hip, M, D, W):
     from webgllm_amd import ops

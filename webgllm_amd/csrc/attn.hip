@@ -1504,57 +1504,123 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(
   }
 }
 
+// half(a - hi.x), half(b - hi.y), the differences exact: v_fma_mix_f32 reads
+// either half of hi as it stands.
+__device__ inline half2v split_rest(half2v hi, float a, float b) {
+  const uint32_t h = __builtin_bit_cast(uint32_t, hi);
+  float x, y;
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(x) : "v"(h), "v"(a));
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(y) : "v"(h), "v"(b));
+  return half2v{(_Float16)x, (_Float16)y};
+}
+
 // The same prompt attention on MFMA (v_mfma_f32_32x32x16_f16, f32
 // accumulation). A wave owns 32 queries (slots of the workgroup's rows x the
-// KV head's G query heads) and walks the keys 32 at a time:
+// KV head's G query heads) and walks the keys 32 KT at a time:
 //  - scores as S^T = K Q^T: A = 32 key rows of the K tile (16-byte pieces,
 //    swizzled as in attn_tile_kernel), B = the wave's queries. The queries
-//    are f32; each is split into hi = half(q) and lo = half(q - hi), two
-//    MFMAs, so the scores keep ~22 bits (the keys are halves already);
+//    are f32 (times log2 e, so the weights are plain powers of two); each is
+//    split into hi = half(q) and lo = half(q - hi), two MFMAs, so the scores
+//    keep ~22 bits (the keys are halves already);
 //  - in that orientation lane i holds 16 keys of query i % 32 (keys
 //    8 (j / 4) + 4 (i / 32) + j % 4 of the tile), so the softmax max and sum
 //    are in-lane plus one exchange between the half-waves;
 //  - weighted values as O^T = V^T P^T: B = the lane's own weights (slice s
 //    of 16 keys = registers 8 s .. 8 s + 7, split hi / lo like the queries),
 //    A = the values of those keys (k-index 8 h + t = key 16 s + 8 (t / 4) +
-//    4 h + t % 4) read from LDS; O^T keeps every output of a lane in its
-//    query, so the online-softmax rescale is per lane.
+//    4 h + t % 4) by transposing LDS loads; O^T keeps every output of a lane
+//    in its query, so the online-softmax rescale is per lane, and is left
+//    out where no lane's maximum moved.
+// The tiles are double buffered: a step's direct-to-LDS loads are issued
+// one step ahead. KW wave groups of QW waves: a group's waves share its
+// tiles, and the groups take the key steps in turn (KW > 1 where the
+// queries alone leave compute units idle), their sums merged in LDS.
+// Bound by the matrix cores (twice the products for the hi / lo splits) and
+// by the vector work a key and query. 2048 rows over 8192 keys, 32 heads
+// over 8 of 128: 1020 us with single-buffered tiles, 2-byte value reads and
+// a mask and rescale every 32 keys; 440 now (1.09 PFLOP/s of products).
 // K and V rows past the block's last visible key (or the cache) are loaded
-// from the chunk's first row instead: stale bits never reach an MFMA.
-template <int HD, int NW>
-__global__ __launch_bounds__(NW * 64) void attn_prefill_mfma_kernel(
+// from the step's first row instead: stale bits never reach an MFMA.
+template <int HD, int QW, int KW, int KT>
+__global__ __launch_bounds__(QW * KW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void attn_prefill_mfma_kernel(
     const float *q, int ldq, int M, int H, int KV, int R, const uint16_t *k_cache,
     const uint16_t *v_cache, const int32_t *pos0_dev, int max_keys, uint16_t *out, int ldo) {
   typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+  typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+  typedef short short4v __attribute__((ext_vector_type(4)));
   typedef float float16v __attribute__((ext_vector_type(16)));
-  constexpr int KP = HD / 8, ROWB = HD * 2, TILE = WK * ROWB, RPI = 64 / KP, NI = WK / RPI;
+  constexpr int KEYS = 32 * KT;  // keys a step
+  constexpr int KP = HD / 8, ROWB = HD * 2, TILE = KEYS * ROWB, RPI = 64 / KP, NI = KEYS / RPI;
   constexpr int KS = HD / 16, DT = HD / 32;
-  __shared__ __align__(16) unsigned char smem[2 * TILE];
+  constexpr int LPW = 2 * NI / QW;  // loads (1 KB) a wave issues a step
+  static_assert(LPW * QW == 2 * NI, "loads split evenly");
+  constexpr int MERGE = 64 * (16 * DT + 2) * 4;  // bytes a merged wave leaves
+  static_assert((KW - 1) * QW * MERGE <= KW * 4 * TILE, "merge area");
+  extern __shared__ __align__(16) unsigned char smem[];  // [KW][2 buffers][K tile, V tile]
   auto swz = [](int r) { return KP == 16 ? (r & 15) : ((r ^ (r >> 3)) & (KP - 1)); };
-  const int kh = blockIdx.x % KV, blk = blockIdx.x / KV;
+  // V rows: 4 rows' 4 neighbouring pieces, which a transposing load takes at
+  // once, land on 16 distinct bank groups
+  auto swzv = [](int r) {
+    return (KP == 16 ? (r & 3) << 2 : (r & 2) << 1) | ((r >> 2) & 3);
+  };
+  // the last rows, which see the most keys, first
+  const int kh = blockIdx.x % KV, blk = (int)(gridDim.x - 1 - blockIdx.x) / KV;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int hh = lane >> 5, c32 = lane & 31;
+  const int wq = wave % QW, kg = wave / QW;
+  const int hh = lane >> 5, c32 = lane & 31, n16 = lane & 15;
   const int G = H / KV, GM = G * R;
   const int m0 = blk * R;
   const int m_last = min(M, m0 + R) - 1;
   const int kvd = KV * HD;
-  const uint32_t sbase = (uint32_t)(uintptr_t)smem;
+  unsigned char *tiles = smem + kg * 4 * TILE;
+  const uint32_t sbase = (uint32_t)(uintptr_t)smem + kg * 4 * TILE;
   const int pos0 = *pos0_dev;
-  // this lane's query (slot qs) and the wave's last visible key
-  const int qs = wave * 32 + c32;
+  // this lane's query (slot qs) and the wave's first and last visible keys
+  const int qs = wq * 32 + c32;
   const int qm = m0 + qs / G;
   const bool qvalid = qs < GM && qm < M;
-  const int q_last = pos0 + qm;  // the last key this query sees
-  const int wlast_slot = min(wave * 32 + 31, GM - 1);
+  const int q_last = min(pos0 + qm, max_keys - 1);  // the last key this query sees
+  const int wlast_slot = min(wq * 32 + 31, GM - 1);
   const int w_row = min(m0 + wlast_slot / G, m_last);
-  const bool w_any = wave * 32 < GM && m0 + (wave * 32) / G <= m_last;
-  const int w_last_key = min(pos0 + w_row, max_keys - 1);
+  const bool w_any = wq * 32 < GM && m0 + (wq * 32) / G <= m_last;
+  const int w_last_key = w_any ? min(pos0 + w_row, max_keys - 1) : -1;
+  // every query of the wave sees the keys up to here
+  const int w_all_key = min(pos0 + m0 + (wq * 32) / G, max_keys - 1);
   const int last_key = min(pos0 + m_last, max_keys - 1);
-  const int nchunks = last_key < 0 ? 0 : last_key / WK + 1;
+  const int steps = last_key < 0 ? 0 : last_key / KEYS + 1;
+  // this lane's pieces of a step's loads: row and byte offset
+  uint32_t off[LPW];
+#pragma unroll
+  for (int i = 0; i < LPW; i++) {
+    const int id = i * QW + wq, r = id % NI * RPI + lane / KP;
+    off[i] = (uint32_t)(r * kvd + (lane % KP ^ (id >= NI ? swzv(r) : swz(r))) * 8) * 2u;
+  }
+  auto issue = [&](int c, int buf) {
+    const int j0 = c * KEYS;
+    const int nk_load = last_key - j0 + 1;  // rows worth loading (>= 1)
+    const uint16_t *kb = k_cache + (int64_t)j0 * kvd + kh * HD;
+    const uint16_t *vb = v_cache + (int64_t)j0 * kvd + kh * HD;
+#pragma unroll
+    for (int i = 0; i < LPW; i++) {
+      const int id = i * QW + wq, ii = id % NI;
+      uint32_t o = off[i];
+      if (nk_load < KEYS) {  // (uniform) rows past the last read row 0
+        const int r = ii * RPI + lane / KP;
+        if (r >= nk_load) o -= (uint32_t)(r * kvd) * 2u;
+      }
+      dma16(id >= NI ? vb : kb, o,
+            __builtin_amdgcn_readfirstlane(sbase + buf * 2 * TILE + (id >= NI ? TILE : 0) +
+                                           ii * 1024));
+    }
+  };
+  const int iters = (steps + KW - 1) / KW;  // of every group
+  if (kg < steps) issue(kg, 0);
   half8 qb_hi[KS], qb_lo[KS];
   {
     const float *qp = q + (int64_t)(qvalid ? qm : 0) * ldq + (int64_t)(kh * G + qs % G) * HD + 8 * hh;
+    constexpr float LOG2E = 1.44269504088896340736f;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
       float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
@@ -1565,9 +1631,10 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_mfma_kernel(
       const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
       for (int t = 0; t < 8; t++) {
-        const _Float16 hi = (_Float16)v[t];
+        const float x = v[t] * LOG2E;
+        const _Float16 hi = (_Float16)x;
         qb_hi[ks][t] = hi;
-        qb_lo[ks][t] = (_Float16)(v[t] - (float)hi);
+        qb_lo[ks][t] = (_Float16)(x - (float)hi);
       }
     }
   }
@@ -1577,87 +1644,160 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_mfma_kernel(
   for (int dt = 0; dt < DT; dt++)
 #pragma unroll
     for (int j = 0; j < 16; j++) o[dt][j] = 0.0f;
-  for (int c = 0; c < nchunks; c++) {
-    const int j0 = c * WK;
-    const int nk_load = min(WK, last_key - j0 + 1);  // rows worth loading (>= 1)
-    for (int i = wave; i < 2 * NI; i += NW) {
-      const bool is_v = i >= NI;
-      const int ii = is_v ? i - NI : i;
-      const int r = ii * RPI + lane / KP;
-      const int slot = lane % KP;
-      const int piece = is_v ? slot : (slot ^ swz(r));
-      const int rr = r < nk_load ? r : 0;
-      dma16((is_v ? v_cache : k_cache) + (int64_t)(j0 + rr) * kvd + kh * HD + piece * 8,
-            __builtin_amdgcn_readfirstlane(sbase + (is_v ? TILE : 0) + ii * 1024));
-    }
+  // this lane's pieces of the operand reads, with swz(r)'s rows folded in: a
+  // K row 32 kt + c32, and the V source row of the transposing loads
+  const int vrow0 = 4 * hh + (n16 >> 2);  // + 32 kt + 16 sl + 8 t
+  for (int it = 0; it < iters; it++) {
+    const int c = it * KW + kg, j0 = c * KEYS;
+    // this step's loads have landed, and every wave of the group is done
+    // with the other buffer
     wait_vm<0>();
-    barrier();
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    if constexpr (QW > 1) barrier();
+    else asm volatile("" ::: "memory");
+    if (c + KW < steps) issue(c + KW, (it + 1) & 1);
+    if (c >= steps || j0 > w_last_key) continue;  // wave-uniform
+    const unsigned char *kt0 = tiles + (it & 1) * 2 * TILE, *vt0 = kt0 + TILE;
+    float16v st[KT];
 #pragma unroll
-    for (int kt = 0; kt < 2; kt++) {
-      const int kb = j0 + 32 * kt;
-      if (!w_any || kb > w_last_key) continue;  // wave-uniform
-      float16v st;
+    for (int kt = 0; kt < KT; kt++)
 #pragma unroll
-      for (int j = 0; j < 16; j++) st[j] = 0.0f;
-      const int r = 32 * kt + c32;
+      for (int j = 0; j < 16; j++) st[kt][j] = 0.0f;
+    half8 ka[2][KT];
+    auto kread = [&](int ks) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ks++) {
-        const half8 ka = *reinterpret_cast<const half8 *>(smem + r * ROWB +
-                                                         (((2 * ks + hh) ^ swz(r)) * 16));
-        st = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qb_hi[ks], st, 0, 0, 0);
-        st = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qb_lo[ks], st, 0, 0, 0);
+      for (int kt = 0; kt < KT; kt++) {
+        const int r = 32 * kt + c32;
+        ka[ks & 1][kt] = *reinterpret_cast<const half8 *>(kt0 + r * ROWB +
+                                                          (((2 * ks + hh) ^ swz(r)) * 16));
       }
-      float p[16];
-      float tmax = -INFINITY;
+    };
+    kread(0);
 #pragma unroll
-      for (int j = 0; j < 16; j++) {
-        const int key = kb + 8 * (j >> 2) + 4 * hh + (j & 3);
-        const bool vis = qvalid && key <= q_last && key < max_keys;
-        p[j] = vis ? st[j] : -INFINITY;
-        tmax = fmaxf(tmax, p[j]);
-      }
-      tmax = fmaxf(tmax, xor32(tmax));
-      const float m_new = fmaxf(m_run, tmax);
-      const float corr = m_new == -INFINITY ? 1.0f : __expf(m_run - m_new);
-      float psum = 0.0f;
+    for (int ks = 0; ks < KS; ks++) {
+      if (ks + 1 < KS) kread(ks + 1);  // under this slice's products
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < 16; j++) {
-        p[j] = p[j] == -INFINITY ? 0.0f : __expf(p[j] - m_new);
-        psum += p[j];
-      }
-      psum += xor32(psum);
-      l_run = l_run * corr + psum;
-      m_run = m_new;
+      for (int kt = 0; kt < KT; kt++)
+        st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[ks & 1][kt], qb_hi[ks], st[kt], 0, 0, 0);
+#pragma unroll
+      for (int kt = 0; kt < KT; kt++)
+        st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[ks & 1][kt], qb_lo[ks], st[kt], 0, 0, 0);
+    }
+    if (j0 + KEYS - 1 > w_all_key) {  // wave-uniform
+      asm volatile("" ::: "memory");  // (stays a branch, not 2 selects a score)
+      const int last = qvalid ? q_last - j0 : -1;
+#pragma unroll
+      for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+        for (int j = 0; j < 16; j++)
+          if (32 * kt + 8 * (j >> 2) + 4 * hh + (j & 3) > last) st[kt][j] = -INFINITY;
+    }
+    float tmax = st[0][0];
+#pragma unroll
+    for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+      for (int j = 0; j < 16; j++) tmax = fmaxf(tmax, st[kt][j]);
+    tmax = fmaxf(tmax, xor32(tmax));
+    const float m_new = fmaxf(m_run, tmax);
+    const float mu = m_new == -INFINITY ? 0.0f : m_new;  // (nothing visible yet: weights 0)
+    if (__ballot(m_new != m_run)) {
+      const float corr = __builtin_amdgcn_exp2f(m_run - mu);
+      l_run *= corr;
 #pragma unroll
       for (int dt = 0; dt < DT; dt++)
 #pragma unroll
         for (int j = 0; j < 16; j++) o[dt][j] *= corr;
+      m_run = m_new;
+    }
+    float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+      for (int j = 0; j < 16; j++) {
+        st[kt][j] = __builtin_amdgcn_exp2f(st[kt][j] - mu);
+        ps[j & 3] += st[kt][j];
+      }
+    float psum = (ps[0] + ps[1]) + (ps[2] + ps[3]);
+    psum += xor32(psum);
+    l_run += psum;
+#pragma unroll
+    for (int kt = 0; kt < KT; kt++)
 #pragma unroll
       for (int sl = 0; sl < 2; sl++) {
         half8 pb_hi, pb_lo;
 #pragma unroll
-        for (int t = 0; t < 8; t++) {
-          const _Float16 hi = (_Float16)p[8 * sl + t];
-          pb_hi[t] = hi;
-          pb_lo[t] = (_Float16)(p[8 * sl + t] - (float)hi);
+        for (int t = 0; t < 8; t += 2) {
+          const half2v hi = {(_Float16)st[kt][8 * sl + t], (_Float16)st[kt][8 * sl + t + 1]};
+          const half2v lo = split_rest(hi, st[kt][8 * sl + t], st[kt][8 * sl + t + 1]);
+          pb_hi[t] = hi.x;
+          pb_hi[t + 1] = hi.y;
+          pb_lo[t] = lo.x;
+          pb_lo[t + 1] = lo.y;
         }
 #pragma unroll
         for (int dt = 0; dt < DT; dt++) {
           half8 va;
 #pragma unroll
-          for (int t = 0; t < 8; t++) {
-            const int vr = 32 * kt + 16 * sl + 8 * (t >> 2) + 4 * hh + (t & 3);
-            va[t] = *reinterpret_cast<const _Float16 *>(smem + TILE + vr * ROWB +
-                                                        (32 * dt + c32) * 2);
+          for (int t2 = 0; t2 < 2; t2++) {
+            // source lane n16 of each 16: row vrow0, dims 32 dt + 16 (their
+            // half of 32) + 4 (n16 % 4) .. + 3; it receives dim 32 dt + c32
+            // of 4 rows
+            const int r = 32 * kt + 16 * sl + 8 * t2 + vrow0;
+            const int col = 32 * dt + (lane & 16) + 4 * (n16 & 3);
+            const unsigned char *at = vt0 + r * ROWB + (((col >> 3) ^ swzv(r)) * 16) + (col & 7) * 2;
+            const half4 h4 = __builtin_bit_cast(
+                half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                           (__attribute__((address_space(3))) short4v *)(uint32_t)(uintptr_t)at));
+#pragma unroll
+            for (int e = 0; e < 4; e++) va[4 * t2 + e] = h4[e];
           }
           o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pb_hi, o[dt], 0, 0, 0);
           o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pb_lo, o[dt], 0, 0, 0);
         }
       }
-    }
-    barrier();  // every wave is done with this chunk's tiles
   }
   wait_vm<0>();
+  if constexpr (KW > 1) {  // the groups' sums meet in LDS, over the tiles
+    const int groups = min(KW, steps);  // that had keys (uniform)
+    auto part = [&](int g) {
+      return reinterpret_cast<float *>(smem) + ((g - 1) * QW + wq) * (MERGE / 4);
+    };
+    if (groups > 1) {
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      barrier();
+      if (kg > 0 && kg < groups) {
+        float *w = part(kg);
+        w[lane] = m_run;
+        w[64 + lane] = l_run;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+            *reinterpret_cast<f4v *>(w + 128 + ((4 * dt + j) * 64 + lane) * 4) =
+                f4v{o[dt][4 * j], o[dt][4 * j + 1], o[dt][4 * j + 2], o[dt][4 * j + 3]};
+      }
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      barrier();
+    }
+    if (kg > 0) return;
+    for (int g = 1; g < groups; g++) {
+      const float *w = part(g);
+      const float m2 = w[lane], mx = fmaxf(m_run, m2);
+      const float mu = mx == -INFINITY ? 0.0f : mx;
+      const float a1 = __builtin_amdgcn_exp2f(m_run - mu), a2 = __builtin_amdgcn_exp2f(m2 - mu);
+      l_run = l_run * a1 + w[64 + lane] * a2;
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const f4v v = *reinterpret_cast<const f4v *>(w + 128 + ((4 * dt + j) * 64 + lane) * 4);
+#pragma unroll
+          for (int e = 0; e < 4; e++) o[dt][4 * j + e] = o[dt][4 * j + e] * a1 + v[e] * a2;
+        }
+      m_run = mx;
+    }
+  }
   if (qvalid) {
     const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
     uint16_t *op = out + (int64_t)qm * ldo + (int64_t)(kh * G + qs % G) * HD;
@@ -1667,6 +1807,23 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_mfma_kernel(
       for (int j = 0; j < 16; j++)
         op[32 * dt + 8 * (j >> 2) + 4 * hh + (j & 3)] = to_h(o[dt][j] * inv);
   }
+}
+
+template <int HD, int QW, int KW, int KT>
+int launch_prefill_mfma(const float *q, int M, int ldq, int H, int KV, const uint16_t *k_cache,
+                        const uint16_t *v_cache, const int32_t *pos0, int max_keys,
+                        uint16_t *out, int ldo, hipStream_t s) {
+  const int R = QW * 32 / (H / KV);  // rows a workgroup
+  const int64_t blocks = (int64_t)KV * ((M + R - 1) / R);
+  WG_REQUIRE(blocks <= 0x7fffffff, "wg_attn_prefill: %d rows", M);
+  constexpr int LDS = KW * 4 * 32 * KT * HD * 2;
+  if (LDS > 64 * 1024) {
+    const int rc = raise_lds((const void *)attn_prefill_mfma_kernel<HD, QW, KW, KT>, LDS);
+    if (rc) return rc;
+  }
+  attn_prefill_mfma_kernel<HD, QW, KW, KT><<<(unsigned)blocks, QW * KW * 64, LDS, s>>>(
+      q, ldq, M, H, KV, R, k_cache, v_cache, pos0, max_keys, out, ldo);
+  return launched("wg_attn_prefill");
 }
 
 }  // namespace
@@ -1866,25 +2023,24 @@ int wg_attn_prefill(const float *q, int32_t M, int32_t ldq, const wg_attn_shape 
   WG_REQUIRE(((uintptr_t)q & 15) == 0 && ldq % 4 == 0,
              "wg_attn_prefill: queries must be 16-byte aligned with a stride of 4k floats");
   hipStream_t s = as_stream(stream);
-  if (const int nw = tuning("attn_prefill_mfma")) {  // waves (32 queries each) a workgroup
-    const int R = nw * 32 / (H / KV);
-    WG_REQUIRE(R >= 1, "wg_attn_prefill: %d query heads a KV head", H / KV);
-    const int64_t blocks = (int64_t)KV * ((M + R - 1) / R);
-    WG_REQUIRE(blocks <= 0x7fffffff, "wg_attn_prefill: %d rows", M);
-#define WG_PF_LAUNCH(NWP)                                                                      \
-  do {                                                                                         \
-    if (hd == 64)                                                                              \
-      attn_prefill_mfma_kernel<64, NWP><<<(unsigned)blocks, NWP * 64, 0, s>>>(                 \
-          q, ldq, M, H, KV, R, k_cache, v_cache, pos0, max_keys, out, ldo);                    \
-    else                                                                                       \
-      attn_prefill_mfma_kernel<128, NWP><<<(unsigned)blocks, NWP * 64, 0, s>>>(                \
-          q, ldq, M, H, KV, R, k_cache, v_cache, pos0, max_keys, out, ldo);                    \
-  } while (0)
-    if (nw == 1) WG_PF_LAUNCH(1);
-    else if (nw == 4) WG_PF_LAUNCH(4);
-    else WG_PF_LAUNCH(2);
+  if (const int form = tuning("attn_prefill_mfma")) {
+    const int G = H / KV, cus = persistent_grid(1 << 30, 1);
+    const int64_t pairs = (int64_t)KV * ((M + 64 / G - 1) / (64 / G));  // of waves of 32 queries
+    // Two waves of queries and two of keys; where those workgroups are fewer
+    // than the compute units, one of queries and four of keys (8B heads: 256
+    // rows at 1000 20 us against 28, 45 at 6000 59 against 102; 512 rows at
+    // 6000, past the line, 135 against 126); from four a compute unit at 128
+    // dims, four of queries (2048 rows over 8192 keys 475 against 508, the
+    // tiles read by half as many groups; 90 against 85 from position 0).
+    const bool few = form == 4 ? pairs < cus : form == 1;
+    const bool wide = hd == 128 && (form == 4 ? pairs >= 4 * (int64_t)cus : form == 3);
+#define WG_PF_LAUNCH(HD, QW, KW, KT)                                                        \
+  launch_prefill_mfma<HD, QW, KW, KT>(q, M, ldq, H, KV, k_cache, v_cache, pos0, max_keys, out, \
+                                      ldo, s)
+    if (hd == 64) return few ? WG_PF_LAUNCH(64, 1, 4, 1) : WG_PF_LAUNCH(64, 2, 2, 2);
+    return few ? WG_PF_LAUNCH(128, 1, 4, 1)
+               : wide ? WG_PF_LAUNCH(128, 4, 1, 1) : WG_PF_LAUNCH(128, 2, 2, 1);
 #undef WG_PF_LAUNCH
-    return launched("wg_attn_prefill");
   }
   const int BR = PF_Q / (H / KV);
   const int64_t blocks = (int64_t)KV * ((M + BR - 1) / BR);
