@@ -386,6 +386,37 @@ def test_attn_prefill_matches_decode_rows(hip, prefill_kernel):
         assert rel_l2(got[m], one[0]) <= 1e-4
 
 
+@pytest.mark.parametrize("H,KV,hd,norm", [(14, 2, 64, False), (32, 8, 64, True),
+                                          (6, 3, 128, True), (32, 8, 128, False)])
+@pytest.mark.parametrize("pos0", [0, 1019])
+def test_head_prep_of_prompt_rows(hip, H, KV, hd, norm, pos0):
+    """Batches of 16 dims a thread: the queries and cache rows of the same
+    rows in two halves, and of rows whose stride is no multiple of 4 floats
+    (both a wave a head), bit for bit, past the cache's end too."""
+    from webgllm_amd import ops
+    rng = np.random.default_rng(H + hd + pos0)
+    M = 65536 // ((H + 2 * KV) * hd // 16) + 5
+    ctx = pos0 + M - 4  # the last 4 rows have no position
+    rope = _t(O.rope_table(1e6, hd, hd, 4096))
+    qkv = _t(rng.standard_normal((M, (H + 2 * KV) * hd)).astype(np.float32))
+    wide = torch.zeros((M, qkv.shape[1] + 1), device="cuda")
+    wide[:, :-1] = qkv
+    w = [_t(rng.uniform(0.5, 1.5, hd).astype(np.float32)) if norm else None for _ in range(2)]
+    shape = ops.attn_shape(H, KV, hd, hd, 1e-6, norm)
+    outs = []
+    for x, step in ((qkv, M), (qkv, M // 2 + 1), (wide, M)):
+        kc = torch.zeros((ctx, KV * hd), dtype=torch.float16, device="cuda")
+        vc = torch.zeros_like(kc)
+        q = torch.cat([ops.head_prep(x[r:r + step], shape, rope,
+                                     _t(np.array([pos0 + r], np.int32)), kc, vc, *w)
+                       for r in range(0, M, step)])
+        outs.append((q, kc, vc))
+    torch.cuda.synchronize()
+    for got in outs[1:]:
+        for x, y in zip(outs[0], got):
+            assert torch.equal(x, y)
+
+
 @pytest.mark.parametrize("waves", [1, 2, 3])
 @pytest.mark.parametrize("H,KV,hd", [(14, 2, 64), (32, 8, 128), (64, 2, 64)])
 @pytest.mark.parametrize("M,pos0", [(1, 0), (9, 22), (17, 47), (33, 63), (70, 190)])

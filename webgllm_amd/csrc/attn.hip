@@ -1504,6 +1504,133 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(
   }
 }
 
+// head_prep_kernel for prompt batches with every dim rotated: HD / 16 threads
+// a head, each with dims 8 c .. 8 c + 7 and their rotation partners HD / 2
+// on, so a head's row moves in 16-byte pieces and a rotation needs no other
+// lane; the same bits (the sum of squares keeps head_norm_inv's order: a
+// chain over dims 32 t + 8 c .. + 7 for each of 4 lanes, which HD = 128's
+// 8 threads pass on between t and t + 1). Bound by memory: 2048 rows of 48
+// heads of 128 (92 MB in and out) took 32 us with a wave a head, 17.6 now.
+template <int HD>
+__global__ __launch_bounds__(256) void head_prep_rows_kernel(
+    const float *qkv, const int32_t *pos0_dev, const float *q_norm, const float *k_norm, int ldq,
+    int H, int KV, int use_norm, float eps, const float *rope, int rope_rows, float *q_out,
+    int ldqo, uint16_t *k_cache, uint16_t *v_cache, int ctx, int M) {
+  constexpr int TPH = HD / 16;  // threads a head (4 or 8)
+  const int slots = H + 2 * KV;
+  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int c = (int)(id % TPH);
+  const int64_t head = id / TPH;
+  const int m = (int)(head / slots), slot = (int)(head % slots);
+  if (m >= M) return;  // (whole heads)
+  const bool is_q = slot < H, is_v = slot >= H + KV;
+  const int pos = *pos0_dev + m;
+  // [0]: dims 8 c .., [1]: their partners
+  float x[2][8], w[2][8];
+  const float *row = qkv + (int64_t)m * ldq + (int64_t)slot * HD + 8 * c;
+  const float *nw = (is_q ? q_norm : k_norm) + 8 * c;
+#pragma unroll
+  for (int p = 0; p < 2; p++)
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const float4 v = *reinterpret_cast<const float4 *>(row + p * (HD / 2) + 4 * u);
+      x[p][4 * u] = v.x;
+      x[p][4 * u + 1] = v.y;
+      x[p][4 * u + 2] = v.z;
+      x[p][4 * u + 3] = v.w;
+      float4 n = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+      if (use_norm && !is_v) n = *reinterpret_cast<const float4 *>(nw + p * (HD / 2) + 4 * u);
+      w[p][4 * u] = n.x;
+      w[p][4 * u + 1] = n.y;
+      w[p][4 * u + 2] = n.z;
+      w[p][4 * u + 3] = n.w;
+    }
+  const bool none = pos < 0 || pos >= ctx || 1024 + (pos >> 10) >= rope_rows;
+  float inv = 1.0f;
+  if (use_norm) {  // (every lane of the wave: the lanes of a head exchange)
+    const int lane = threadIdx.x & 63, head0 = lane - c;
+    float part = 0.0f;
+    if constexpr (HD == 64) {
+#pragma unroll
+      for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) part = __builtin_fmaf(x[p][e], x[p][e], part);
+    } else {
+      // t = 0, 2 on threads c < 4, t = 1, 3 on threads c + 4
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        if (t) part = __shfl(part, head0 + (c ^ 4), 64);
+#pragma unroll
+        for (int e = 0; e < 8; e++) part = __builtin_fmaf(x[t >> 1][e], x[t >> 1][e], part);
+      }
+      // the chains that began at t = 0 ended on threads 4 .. 7
+    }
+    constexpr int END = HD == 64 ? 0 : 4;
+    const float total = (__shfl(part, head0 + END, 64) + __shfl(part, head0 + END + 1, 64)) +
+                        (__shfl(part, head0 + END + 2, 64) + __shfl(part, head0 + END + 3, 64));
+    inv = head_norm_inv(total, HD, eps);
+  }
+  const int kvd = KV * HD;
+  if (is_v) {
+    if (none) return;
+    uint16_t *o = v_cache + (int64_t)pos * kvd + (int64_t)(slot - H - KV) * HD + 8 * c;
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+      *reinterpret_cast<uint4 *>(o + p * (HD / 2)) =
+          make_uint4(to_h(x[p][0]) | (uint32_t)to_h(x[p][1]) << 16,
+                     to_h(x[p][2]) | (uint32_t)to_h(x[p][3]) << 16,
+                     to_h(x[p][4]) | (uint32_t)to_h(x[p][5]) << 16,
+                     to_h(x[p][6]) | (uint32_t)to_h(x[p][7]) << 16);
+    return;
+  }
+  if (none && !is_q) return;
+  float r[2][8];
+  if (none) {  // a row past the cache has no position: its query is zero
+#pragma unroll
+    for (int e = 0; e < 8; e++) r[0][e] = r[1][e] = 0.0f;
+  } else {
+    const float *r_lo = rope + (int64_t)(pos & 1023) * HD + 8 * c;
+    const float *r_hi = rope + (int64_t)(1024 + (pos >> 10)) * HD + 8 * c;
+    const float scale = is_q ? 1.0f / sqrtf((float)HD) : 1.0f;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const float4 c1 = *reinterpret_cast<const float4 *>(r_lo + 4 * u);
+      const float4 s1 = *reinterpret_cast<const float4 *>(r_lo + HD / 2 + 4 * u);
+      const float4 c2 = *reinterpret_cast<const float4 *>(r_hi + 4 * u);
+      const float4 s2 = *reinterpret_cast<const float4 *>(r_hi + HD / 2 + 4 * u);
+      const float fc1[4] = {c1.x, c1.y, c1.z, c1.w}, fs1[4] = {s1.x, s1.y, s1.z, s1.w};
+      const float fc2[4] = {c2.x, c2.y, c2.z, c2.w}, fs2[4] = {s2.x, s2.y, s2.z, s2.w};
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int d = 4 * u + e;
+        const float a = x[0][d] * (use_norm ? inv * w[0][d] : 1.0f);
+        const float b = x[1][d] * (use_norm ? inv * w[1][d] : 1.0f);
+        r[0][d] = rope_rotate(a, b, true, fc1[e], fs1[e], fc2[e], fs2[e]);
+        r[1][d] = rope_rotate(b, a, false, fc1[e], fs1[e], fc2[e], fs2[e]);
+        if (is_q) {
+          r[0][d] *= scale;
+          r[1][d] *= scale;
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < 2; p++) {
+    if (is_q) {
+      float *o = q_out + (int64_t)m * ldqo + (int64_t)slot * HD + 8 * c + p * (HD / 2);
+      *reinterpret_cast<float4 *>(o) = make_float4(r[p][0], r[p][1], r[p][2], r[p][3]);
+      *reinterpret_cast<float4 *>(o + 4) = make_float4(r[p][4], r[p][5], r[p][6], r[p][7]);
+    } else {
+      uint16_t *o = k_cache + (int64_t)pos * kvd + (int64_t)(slot - H) * HD + 8 * c + p * (HD / 2);
+      *reinterpret_cast<uint4 *>(o) =
+          make_uint4(to_h(r[p][0]) | (uint32_t)to_h(r[p][1]) << 16,
+                     to_h(r[p][2]) | (uint32_t)to_h(r[p][3]) << 16,
+                     to_h(r[p][4]) | (uint32_t)to_h(r[p][5]) << 16,
+                     to_h(r[p][6]) | (uint32_t)to_h(r[p][7]) << 16);
+    }
+  }
+}
+
 // half(a - hi.x), half(b - hi.y), the differences exact: v_fma_mix_f32 reads
 // either half of hi as it stands.
 __device__ inline half2v split_rest(half2v hi, float a, float b) {
@@ -1998,6 +2125,23 @@ int wg_head_prep(const float *qkv, int32_t M, int32_t ldq, const wg_attn_shape *
   int slots = sh->heads + 2 * sh->kv_heads;
   WG_REQUIRE(ldq >= slots * sh->head_dim && ldqo >= sh->heads * sh->head_dim,
              "wg_head_prep: strides too small");
+  const int hd = sh->head_dim;
+  const uintptr_t ptrs = (uintptr_t)qkv | (uintptr_t)q_norm | (uintptr_t)k_norm |
+                         (uintptr_t)rope | (uintptr_t)q_out | (uintptr_t)k_cache |
+                         (uintptr_t)v_cache;
+  // Few rows wait on memory round trips, which a wave a head takes fewer of
+  // (131 rows of 18 heads of 64: 3.0 us against 4.2); 16 dims a thread where
+  // that gives every compute unit a workgroup and the 16-byte pieces are
+  // aligned.
+  const int64_t threads = (int64_t)M * slots * (hd / 16);
+  if (threads >= 256 * (int64_t)persistent_grid(1 << 30, 1) && (hd == 64 || hd == 128) &&
+      sh->rotated_dims == hd && (ptrs & 15) == 0 && ldq % 4 == 0 && ldqo % 4 == 0) {
+    auto kernel = hd == 64 ? head_prep_rows_kernel<64> : head_prep_rows_kernel<128>;
+    kernel<<<(unsigned)((threads + 255) / 256), 256, 0, as_stream(stream)>>>(
+        qkv, pos0, q_norm, k_norm, ldq, sh->heads, sh->kv_heads, sh->use_norm, sh->eps, rope,
+        rope_rows, q_out, ldqo, k_cache, v_cache, ctx, M);
+    return launched("wg_head_prep");
+  }
   head_prep_kernel<<<dim3(slots, M), 64, 0, as_stream(stream)>>>(
       qkv, pos0, q_norm, k_norm, ldq, sh->heads, sh->kv_heads, sh->head_dim, sh->use_norm,
       sh->rotated_dims, sh->eps, rope, rope_rows, q_out, ldqo, k_cache, v_cache, ctx);
