@@ -117,6 +117,32 @@ def test_gemm_every_tile(hip, fmt, tile):
     assert e16 <= 1e-5
 
 
+@pytest.mark.parametrize("tile", [4, 5, 6, 7])
+@pytest.mark.parametrize("fmt", ["q4_0", "nbits", "q4_k_rowgroup", "q8"])
+def test_gemm_wave_groups(hip, fmt, tile):
+    """Each tile whose wave groups split K: one step (all groups but one
+    without any), a step count no group count divides, partial row tiles, a
+    residual in place; the SwiGLU form gives the bits of the plain one."""
+    from webgllm_amd import lib as L, ops
+    L.tuning_set("gemm_tile", tile)
+    try:
+        for M, N, K in ((1, 128, 256), (33, 384, 768), (70, 256, 2304)) + \
+                (() if fmt.startswith("q4_k") else ((65, 128, 64), (40, 128, 576))):
+            m = _matrix(fmt, N, K, seed=tile + K)
+            e, e16 = _check(m, M, seed=M, residual=K == 768)
+            assert e <= 1e-3 and e16 <= 1e-5, (M, N, K)
+            a = torch.randn((M, K), device="cuda").half()
+            rs = torch.rand(M, device="cuda") + 0.5
+            gu = ops.gemm(m, a, row_scale=rs)
+            # stored rows (gate, gate, up, up) to gate columns, then up columns
+            order = torch.arange(N, device="cuda").view(-1, 2, 2).transpose(0, 1).reshape(-1)
+            want = ops.swiglu(gu[:, order].contiguous())
+            got = ops.gemm_swiglu(m, a, row_scale=rs)
+            assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (M, N, K)
+    finally:
+        L.tuning_set("gemm_tile", 0)
+
+
 def test_gemm_column_map(hip):
     """col_of sends stored row n to output column col_of[n]: the mapped
     product equals the plain one with its columns permuted (bit for bit);

@@ -40,8 +40,11 @@
 //  - workgroups on one XCD (ids equal mod 8, as the dispatcher deals them
 //    round-robin) take the M tiles of one weight tile one after another, so
 //    it is read from HBM once into that XCD's L2;
-//  - when the tiles are fewer than the compute units (M = 512 at N = 4096
-//    gives 128 tiles of 128 x 128), K is split KS ways (2 or 4): each
+//  - short prompts and small matrices run smaller tiles, 8 waves in 2 to 8
+//    groups that take a part of K each with a ring of their own and add their
+//    sums in LDS;
+//  - elsewhere, when the tiles are fewer than the compute units (M = 512 at
+//    K = 14336, N = 4096 gives 128 tiles of 128 x 128), K is split KS ways (2 or 4): each
 //    workgroup runs one K range of one tile; the splits' float32 sums meet
 //    in a fixed pairwise tree (coherent stores and loads, counters put back
 //    to zero by their last arriver), and the tile's last workgroup runs the
@@ -143,11 +146,12 @@ struct Stage {
 
 // Waves a SIMD holds at once, as the LDS ring allows (160 KB a compute
 // unit, 4 SIMDs): the register budget the compiler may spend.
-template <int ZK, int BM, int BN, int S, int NWV>
+template <int ZK, int BM, int BN, int S, int NWV, int KG = 1>
 constexpr int gemm_waves_per_simd() {
-  constexpr int stage = BM * 128 + Stage<ZK, BN>::WQ + Stage<ZK, BN>::WS + Stage<ZK, BN>::WZ;
+  constexpr int stage =
+      KG * (BM * 128 + Stage<ZK, BN>::WQ + Stage<ZK, BN>::WS + Stage<ZK, BN>::WZ);
   constexpr int wgs = (160 * 1024) / (S * stage);
-  constexpr int w = (wgs * NWV + 3) / 4;
+  constexpr int w = (wgs * NWV * KG + 3) / 4;
   return w < 1 ? 1 : w > 8 ? 8 : w;
 }
 
@@ -186,9 +190,14 @@ __device__ inline bool count_in(int *count, int expect) {
 // + 1) and C is a half output [M][ldc] of N / 2 columns: half(silu(gate) *
 // up), as REDUCE_SWIGLU (src/gpu/kernels.ts:1066-1077) computes it from
 // the float32 sums.
-template <int ZK, int BM, int BN, int S, int WGM, int WGN, bool SW = false, bool PP = false>
-__global__ __launch_bounds__(WGM * WGN * 64) __attribute__((amdgpu_waves_per_eu(
-    1, gemm_waves_per_simd<ZK, BM, BN, S, WGM * WGN>()))) void gemm_q4_kernel(const uint8_t *__restrict__ quants,
+// KG > 1: that many groups of WGM x WGN waves, each with a ring of its own,
+// take a KG-th of K, their sums meeting in LDS (small matrices and short
+// prompts: the waves a compute unit needs, without splits that meet through
+// memory).
+template <int ZK, int BM, int BN, int S, int WGM, int WGN, bool SW = false, bool PP = false,
+          int KG = 1>
+__global__ __launch_bounds__(WGM * WGN * KG * 64) __attribute__((amdgpu_waves_per_eu(
+    1, gemm_waves_per_simd<ZK, BM, BN, S, WGM * WGN, KG>()))) void gemm_q4_kernel(const uint8_t *__restrict__ quants,
                                                       const uint16_t *__restrict__ scales,
                                                       const void *__restrict__ zeros,
                                                       const uint16_t *__restrict__ A, int lda,
@@ -210,10 +219,12 @@ __global__ __launch_bounds__(WGM * WGN * 64) __attribute__((amdgpu_waves_per_eu(
   constexpr int QSTEP = RGP * 16;  // weight bytes a row group moves a step
   constexpr int IQ = QP > 64 * NWV ? QP / (64 * NWV) : 1;  // nibble loads a wave issues
   constexpr int NW = IA + IQ + 1 + (ZK == WG_ZERO_U8 ? 1 : 0);  // loads a wave issues a stage
-  extern __shared__ __align__(16) unsigned char smem[];
+  static_assert(KG == 1 || !PP, "wave groups run in lock-step");
+  extern __shared__ __align__(16) unsigned char smem_all[];
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((tid >> 6) / NWV);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) - kg * NWV;  // of its group
   const int wm = wave / WGN, wn = wave % WGN, h = lane >> 5;
   // the ping-pong group: waves 0-3 and 4-7 (wave w runs on SIMD w % 4)
   static_assert(!PP || NWV == 8, "the ping-pong schedule pairs 8 waves");
@@ -237,7 +248,11 @@ __global__ __launch_bounds__(WGM * WGN * 64) __attribute__((amdgpu_waves_per_eu(
   }
   const int m0 = tm * BM, n0 = tn * BN, g0 = n0 / 4;
   // this workgroup's K steps of 64: KT of them from step kb
-  const int B = K / 32, KT = K / 64 / ks, kb = split * KT;
+  const int B = K / 32, KA = K / 64 / ks;
+  const int kb = KG == 1 ? split * KA : KA * kg / KG;
+  const int KT = KG == 1 ? KA : KA * (kg + 1) / KG - kb;
+  const int KMAX = KG == 1 ? KT : (KA + KG - 1) / KG;  // of any group
+  unsigned char *smem = smem_all + kg * S * STAGE;
   const uint32_t sbase = (uint32_t)(uintptr_t)smem;
 
   // This wave's loads of a step: per-lane byte offsets fixed for the whole
@@ -247,7 +262,9 @@ __global__ __launch_bounds__(WGM * WGN * 64) __attribute__((amdgpu_waves_per_eu(
   constexpr int PWQ = QP > 64 * NWV ? 64 : QP / NWV;  // lanes a nibble load
   static_assert(PWQ >= 1 && IQ * NWV * PWQ == QP, "nibble pieces");
   constexpr int NSC = BN / 4, PIECES = ZK == WG_ZERO_F16 ? 2 * NSC : NSC, PWS = PIECES / NWV;
-  static_assert(PWS >= 1 && PWS * NWV == PIECES && NSC % PWS == 0, "scale pieces");
+  // (one wave takes both arrays' pieces: its lanes' bases differ)
+  constexpr bool MIXED = NSC % PWS != 0;
+  static_assert(PWS >= 1 && PWS * NWV == PIECES && (!MIXED || NWV == 1), "scale pieces");
   constexpr int PWZ = ZK == WG_ZERO_U8 ? 2 * BN / 4 / NWV : 1;
   static_assert(ZK != WG_ZERO_U8 || (PWZ >= 1 && PWZ * NWV * 4 == 2 * BN), "zero-point pieces");
   uint32_t off_a[IA];
@@ -265,7 +282,7 @@ __global__ __launch_bounds__(WGM * WGN * 64) __attribute__((amdgpu_waves_per_eu(
     off_q[i] = (uint32_t)(((int64_t)(g0 + qq / RGP) * B) * (QSTEP / 2) + (qq % RGP) * 16);
   }
   const int qs = wave * PWS + lane;
-  const bool s_is_zero = wave * PWS >= NSC;  // wave-uniform
+  const bool s_is_zero = (MIXED ? qs : wave * PWS) >= NSC;  // wave-uniform unless MIXED
   const uint32_t off_s = (uint32_t)((int64_t)(g0 + (s_is_zero ? qs - NSC : qs)) * B * 8);
   const int qz = wave * PWZ + lane;
   const uint32_t off_z = (uint32_t)(((int64_t)(g0 + (qz >> 1)) * B) * 4 + (qz & 1) * 4);
@@ -283,9 +300,11 @@ __global__ __launch_bounds__(WGM * WGN * 64) __attribute__((amdgpu_waves_per_eu(
       if (lane < PWQ)
         dma16(quants + kt * QSTEP, off_q[i],
               __builtin_amdgcn_readfirstlane(base + A_BYTES + (i * NWV + wave) * PWQ * 16));
-    if (lane < PWS)
-      dma16(s_base + kt * 16, off_s,
-            __builtin_amdgcn_readfirstlane(base + A_BYTES + WQ + wave * PWS * 16));
+    if (lane < PWS) {
+      const uint32_t to = __builtin_amdgcn_readfirstlane(base + A_BYTES + WQ + wave * PWS * 16);
+      if constexpr (MIXED) dma16((const void *)(s_base + kt * 16 + off_s), to);
+      else dma16(s_base + kt * 16, off_s, to);
+    }
     if constexpr (ZK == WG_ZERO_U8) {  // 8 zero-point bytes a row group, 4 at a time
       if (lane < PWZ)
         dma4((const uint8_t *)zeros + kt * 8, off_z,
@@ -371,15 +390,16 @@ __global__ __launch_bounds__(WGM * WGN * 64) __attribute__((amdgpu_waves_per_eu(
     if (s < KT) issue(s, s);
   // Unrolled by S: a step's stage is a constant, so its LDS addresses are
   // immediate offsets.
-  for (int k0 = 0; k0 < KT; k0 += S) {
+  for (int k0 = 0; k0 < KMAX; k0 += S) {
 #pragma unroll
   for (int ss = 0; ss < S; ss++) {
     const int kt = k0 + ss;
-    if (kt >= KT) break;
+    if (kt >= KMAX) break;
     // this wave's loads of step kt have landed (younger stages may fly on)
     if (kt + S - 2 < KT) wait_vm<NW * (S - 2)>();
     else wait_vm<0>();
     barrier();  // every wave's have, and every wave is done with step kt - 1
+    if (KG > 1 && kt >= KT) break;  // (a group one step short: KMAX - 1 of them)
     const unsigned char *st = smem + ss * STAGE;
     if constexpr (PP) {
       // Two wave groups half a step apart, one wave of each on every SIMD:
@@ -416,7 +436,43 @@ __global__ __launch_bounds__(WGM * WGN * 64) __attribute__((amdgpu_waves_per_eu(
     if (group && KT > 0) amfmas(smem + ((KT - 1) % S) * STAGE);  // group 1's last step
   }
 
-  if (ks > 1) {
+  if constexpr (KG > 1) {
+    // The groups' sums meet over the rings, added in the groups' order; a
+    // fragment (wave, t, u) is 16 floats a lane in four 16-byte pieces.
+    reads_done();
+    __syncthreads();
+    float *red = reinterpret_cast<float *>(smem_all) + 4 * lane;
+    auto at = [&](int g, int t, int u, int j4) {
+      return ((((g - 1) * NWV + wave) * MT + t) * NT + u) * 1024 + j4 * 256;
+    };
+    static_assert((KG - 1) * NWV * MT * NT * 4096 <= KG * S * STAGE, "sums fit the rings");
+    if (kg > 0) {
+#pragma unroll
+      for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int u = 0; u < NT; u++)
+#pragma unroll
+          for (int j4 = 0; j4 < 4; j4++)
+            *reinterpret_cast<f4v *>(red + at(kg, t, u, j4)) =
+                f4v{acc[t][u][4 * j4], acc[t][u][4 * j4 + 1], acc[t][u][4 * j4 + 2],
+                    acc[t][u][4 * j4 + 3]};
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int g = 1; g < KG; g++)
+#pragma unroll
+      for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int u = 0; u < NT; u++)
+#pragma unroll
+          for (int j4 = 0; j4 < 4; j4++) {
+            const f4v v = *reinterpret_cast<const f4v *>(red + at(g, t, u, j4));
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[t][u][4 * j4 + e] += v[e];
+          }
+  }
+  if (KG == 1 && ks > 1) {
     // The splits' sums meet in a fixed pairwise tree: at level l, group g
     // (the 2^l splits from g 2^l) publishes its sum in slot 2 ks - 2 ks /
     // 2^l + g, and the last of each pair of groups adds its partner's. An
@@ -645,6 +701,25 @@ int expand_space(hipStream_t s, size_t count, uint16_t **out) {
   return WG_OK;
 }
 
+template <int ZK, int BM, int BN, int S, int WGM, int WGN, int KG, bool SW>
+int launch_groups(const wg_q4_matrix *w, const uint16_t *A, int M, int lda, float *C, int ldc,
+                  const float *residual, int ldr, const float *row_scale, const int32_t *col_of,
+                  hipStream_t s) {
+  constexpr int STAGE = BM * 128 + Stage<ZK, BN>::WQ + Stage<ZK, BN>::WS + Stage<ZK, BN>::WZ;
+  constexpr size_t LDS = (size_t)KG * S * STAGE;
+  static_assert(LDS <= 160 * 1024, "LDS");
+  auto kernel = gemm_q4_kernel<ZK, BM, BN, S, WGM, WGN, SW, false, KG>;
+  if (LDS > 64 * 1024) {
+    const int rc = raise_lds((const void *)kernel, (int)LDS);
+    if (rc) return rc;
+  }
+  const int tiles = ((M + BM - 1) / BM) * (w->N / BN);
+  kernel<<<tiles, WGM * WGN * KG * 64, LDS, s>>>(
+      (const uint8_t *)w->quants, (const uint16_t *)w->scales, w->zeros, A, lda, C, ldc,
+      residual, ldr, row_scale, col_of, M, w->N, w->K, 1, nullptr, nullptr);
+  return launched(SW ? "wg_q4_gemm_swiglu" : "wg_q4_gemm");
+}
+
 template <int ZK, int BM, int BN, int S, int WGM = 2, int WGN = 2, bool SW = false,
           bool PP = false>
 int launch_tiles(const wg_q4_matrix *w, const uint16_t *A, int M, int lda, float *C, int ldc,
@@ -698,11 +773,40 @@ int launch(const wg_q4_matrix *w, const uint16_t *A, int M, int lda, float *C, i
   // The knob gemm_tile forces one (1: 64 x 128, 2: 128 x 128, 3: 128 x 256).
   const int cus = persistent_grid(1 << 30, 1);
   int t = tuning("gemm_tile");
+  // Wave groups (4: 64 x 128 and 2 groups, 5: 64 x 64 and 4, 6: 32 x 32 and
+  // 8, 7: 32 x 64 and 4): the smallest tile whose workgroups all run at once
+  // (7's rings leave room for two a compute unit but for 8-bit weights), so
+  // that no weight waits for a second round and no sum goes through memory.
+  // Microseconds, with groups / the forms below: 131 rows of 896 -> 1152 6.8
+  // / 12.5 (6), 896 -> 9728 10.7 / 15.0 (4), 4864 -> 896 12.4 / 23.9 (6); 45
+  // rows, 8-bit, 2048 -> 16384 13.6 / 20.2 (5), 8192 -> 2048 15.8 / 23.0
+  // (6); 512 rows of 2048 -> 2048 13.4 / 28.8 (7), 4096 -> 4096 40.7 / 51.4
+  // (4). Past those workgroups they are slower (512 rows of 896 -> 9728 28.9
+  // / 22.7), and past 8192 deep, where the loop outweighs the splits'
+  // meeting, no faster (131 rows of 14336 -> 4096 63 / 60; 6, with 45 rows,
+  // 32.9 / 45.0). Rows under 768 deep (12 steps) keep the forms below too:
+  // the groups would save them 4 of 8 to 10 us, but models that narrow are
+  // tests', whose greedy picks follow the order of the sums.
+  if (t == 0 && w->K >= 768 && tuning("gemm_splits") <= 1) {  // (2 and more force splits)
+    const int64_t m32 = (M + 31) / 32, m64 = (M + 63) / 64;
+    const bool shallow = w->K <= 8192;
+    if (m32 * (w->N / 32) <= cus) t = 6;
+    else if (shallow && m32 * (w->N / 64) <= (ZK == Q8 ? 1 : 2) * cus) t = 7;
+    else if (shallow && m64 * (w->N / 64) <= cus) t = 5;
+    else if (shallow && w->N % 128 == 0 && m64 * (w->N / 128) <= cus) t = 4;
+  }
   if (t == 0) {
     if (w->N % 256 == 0 && (int64_t)((M + 127) / 128) * (w->N / 256) * 4 >= (int64_t)cus * 3) t = 3;
     else if (M >= 512 && w->N % 128 == 0) t = 2;
     else if (w->N % 128 == 0) t = 1;
   }
+#define WG_GROUPS(BM, BN, S, WN, KG) \
+  launch_groups<ZK, BM, BN, S, 1, WN, KG, SW>(w, A, M, lda, C, ldc, residual, ldr, row_scale, col_of, s)
+  if (t == 4 && w->N % 128 == 0) return WG_GROUPS(64, 128, 4, 4, 2);
+  if (t == 5) return WG_GROUPS(64, 64, 3, 2, 4);
+  if (t == 6) return WG_GROUPS(32, 32, 3, 1, 8);
+  if (t == 7) return WG_GROUPS(32, 64, 3, 2, 4);
+#undef WG_GROUPS
   if (t == 3 && w->N % 256 == 0) {
     if (tuning("gemm_pingpong"))
       return launch_tiles<ZK, 128, 256, 3, 1, 8, SW, true>(w, A, M, lda, C, ldc, residual, ldr,
