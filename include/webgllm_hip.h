@@ -579,6 +579,61 @@ int wg_head_prep(const float *qkv, int32_t M, int32_t ldq, const wg_attn_shape *
 int wg_attn_prefill(const float *q, int32_t M, int32_t ldq, const wg_attn_shape *shape,
                     const uint16_t *k_cache, const uint16_t *v_cache, const int32_t *pos0,
                     int32_t max_keys, uint16_t *out, int32_t ldo, void *stream);
+
+/* One layer of a prompt batch: a short-conv layer (conv_width > 0: in is
+ * in_proj, out out_proj) or an attention layer (in is q|k|v with its column
+ * map, or NULL, and out the o projection). q_norm and k_norm as wg_head_prep
+ * takes them. */
+typedef struct wg_prefill_layer {
+  const float *op_norm;
+  const float *ffn_norm;
+  wg_q4_matrix in;
+  wg_q4_matrix out;
+  wg_q4_matrix gate_up; /* in the SwiGLU row order */
+  wg_q4_matrix down;
+  const int32_t *col_of;
+  const float *q_norm;
+  const float *k_norm;
+  uint16_t *k_cache;
+  uint16_t *v_cache;
+  const float *conv_taps;
+  float *conv_state;
+  int32_t conv_width;
+} wg_prefill_layer;
+
+/* The batch: M rows of width D at positions *pos + m, caches of ctx rows;
+ * h [M][D] the residual stream, updated; the others scratch of M rows (x16,
+ * c16 of D halves, rs of 1 float, bcx of 3 D, qkv of q|k|v and q of the
+ * heads' floats, att16 of the heads' halves, ff16 of F halves). */
+typedef struct wg_prefill_batch {
+  int32_t M;
+  int32_t D;
+  int32_t F;
+  float eps;
+  wg_attn_shape attn;
+  const float *rope;
+  int32_t rope_rows;
+  int32_t ctx;
+  const int32_t *pos;
+  float *h;
+  uint16_t *x16;
+  float *rs;
+  float *bcx;
+  uint16_t *c16;
+  float *qkv;
+  float *q;
+  uint16_t *att16;
+  uint16_t *ff16;
+} wg_prefill_batch;
+
+/* A prompt batch through `count` layers: for each, wg_norm_to_h2, wg_q4_gemm
+ * of `in` (times the row scale), wg_short_conv or wg_head_prep and
+ * wg_attn_prefill, wg_q4_gemm of `out` into h (Engine.forwardBatch,
+ * engine.ts:4969-5234), wg_norm_to_h2, wg_q4_gemm_swiglu and wg_q4_gemm of
+ * `down` into h: those calls in turn, the first error returned. */
+int wg_prefill_layers(const wg_prefill_layer *layers, int32_t count,
+                      const wg_prefill_batch *batch, void *stream);
+
 /* Decode / verify attention (scores, attend, attendPanel + attendPanelCombine,
  * kernels.ts:2386-2579, :2803-3027): row m's query at position *pos0 + m
  * attends keys 0..*pos0 + m (causal) of its KV head; half output. max_keys

@@ -399,3 +399,26 @@ def test_verify_grows_the_cache(hip, family):
     tokens, kept2 = eng2.verify_drafts(token, fed)
     assert eng2.kv_positions == 2048
     assert kept2 == kept and tokens == written
+
+
+@pytest.mark.parametrize("family", sorted(FAMILIES))
+def test_prompt_layers_in_one_call_equal_the_calls_in_turn(hip, family):
+    """A prompt's layers from the native call and, with a probe set, one
+    operation at a time: the same logits, caches and states bit for bit, on a
+    new sequence, a continued one and after the caches have grown."""
+    outs = []
+    for probe in (None, lambda *a: None):
+        eng, _ = _pair(family, seed=5, ctx=1024)
+        rng = np.random.default_rng(1)
+        got = []
+        for n in (9, 40, 300):
+            eng.probe = probe
+            picks = eng.forward(_prompt(rng, n, eng.shape.vocab))
+            eng.probe = None
+            got += [picks, eng.logits[:len(picks)].clone()]
+        for i in sorted(eng.k_cache):
+            got += [eng.k_cache[i][:eng.position], eng.v_cache[i][:eng.position]]
+        outs.append(got + [eng.state[i] for i in sorted(eng.state)])
+    torch.cuda.synchronize()
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)

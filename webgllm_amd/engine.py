@@ -511,6 +511,34 @@ class Engine:
             self._cols[key] = torch.tensor(order, dtype=torch.int32, device=self.device)
         return self._cols[key]
 
+    def _prefill_layers(self):
+        """The layers as wg_prefill_layers takes them, made for each batch
+        from what the engine holds (caches grow, weights may be replaced)."""
+        s, f32, p = self.shape, torch.float32, ops._p
+        layers = (L.PrefillLayer * len(self.w.layers))()
+        for i, lw in enumerate(self.w.layers):
+            a = layers[i]
+            a.op_norm, a.ffn_norm = p(ops._dev(lw["op_norm"], f32)), p(ops._dev(lw["ffn_norm"], f32))
+            a.gate_up, a.down = lw["gate_up"].prompt_desc(), lw["down"].prompt_desc()
+            if s.layer_type(i) == "conv":
+                a.in_, a.out = lw["in_proj"].prompt_desc(), lw["out_proj"].prompt_desc()
+                a.conv_taps, a.conv_state = p(ops._dev(lw["taps"])), p(self.state[i])
+                a.conv_width = s.conv_kernel
+            else:
+                a.in_, a.out = lw["qkv"].prompt_desc(), lw["o"].prompt_desc()
+                a.col_of = p(self._col_of(lw["qkv"]))
+                a.q_norm, a.k_norm = p(lw.get("q_norm")), p(lw.get("k_norm"))
+                a.k_cache, a.v_cache = p(self.k_cache[i]), p(self.v_cache[i])
+        return layers
+
+    def _prefill_batch(self, M: int) -> "L.PrefillBatch":
+        s, b, p = self.shape, self._pre_buffers(), ops._p
+        ctx = next((c.shape[0] for c in self.k_cache.values()), 0)
+        return L.PrefillBatch(M, s.hidden, s.intermediate, s.eps, self.attn, p(self.rope),
+                              self.rope.shape[0], ctx, p(self.pos),
+                              *(p(b[n]) for n in ("h", "x16", "rs", "bcx", "c16", "qkv", "q",
+                                                  "att16", "ff16")))
+
     def _prefill_rows(self, M: int) -> None:
         """A prompt batch of M rows (pre ids[:M] at positions pos ..) through
         the GEMMs on MFMA, as the reference's forwardBatch takes batches larger
@@ -518,11 +546,15 @@ class Engine:
         attention plan for a prompt, :6359-6630). A norm's output is the
         reference's prescaled half(h w / 32), its 32 / RMS the GEMM's row
         scale, as in the few-token path; the caches and conv states advance;
-        no head here (_prefill_head)."""
+        no head here (_prefill_head). The layers run from one native call, or,
+        for a probe between them, from here."""
         s, w, b = self.shape, self.w, self._pre_buffers()
         D = s.hidden
         h, x16, rs = b["h"][:M], b["x16"][:M], b["rs"][:M]
         ops.embed(w.embedding, b["ids"][:M], out=h)
+        if not self.probe:
+            ops.prefill_layers(self._prefill_layers(), self._prefill_batch(M))
+            return
         for i, lw in enumerate(w.layers):
             ops.norm_to_h2(h, lw["op_norm"], s.eps, x16, rs)
             if s.layer_type(i) == "conv":

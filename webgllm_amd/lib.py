@@ -71,6 +71,25 @@ class AttnShape(C.Structure):
                 ("rotated_dims", C.c_int32), ("eps", C.c_float), ("use_norm", C.c_int32)]
 
 
+class PrefillLayer(C.Structure):
+    """wg_prefill_layer."""
+    _fields_ = [("op_norm", C.c_void_p), ("ffn_norm", C.c_void_p), ("in_", Q4MatrixDesc),
+                ("out", Q4MatrixDesc), ("gate_up", Q4MatrixDesc), ("down", Q4MatrixDesc),
+                ("col_of", C.c_void_p), ("q_norm", C.c_void_p), ("k_norm", C.c_void_p),
+                ("k_cache", C.c_void_p), ("v_cache", C.c_void_p), ("conv_taps", C.c_void_p),
+                ("conv_state", C.c_void_p), ("conv_width", C.c_int32)]
+
+
+class PrefillBatch(C.Structure):
+    """wg_prefill_batch."""
+    _fields_ = [("M", C.c_int32), ("D", C.c_int32), ("F", C.c_int32), ("eps", C.c_float),
+                ("attn", AttnShape), ("rope", C.c_void_p), ("rope_rows", C.c_int32),
+                ("ctx", C.c_int32), ("pos", C.c_void_p), ("h", C.c_void_p), ("x16", C.c_void_p),
+                ("rs", C.c_void_p), ("bcx", C.c_void_p), ("c16", C.c_void_p),
+                ("qkv", C.c_void_p), ("q", C.c_void_p), ("att16", C.c_void_p),
+                ("ff16", C.c_void_p)]
+
+
 class DeltaShape(C.Structure):
     """wg_delta_shape."""
     _fields_ = [("heads", C.c_int32), ("key_dim", C.c_int32), ("value_dim", C.c_int32)]
@@ -192,6 +211,8 @@ def load():
                                    P, P, I32, P]),
         "wg_attn_scratch_bytes": (SZ, [I32, I32, I32, I32]),
         "wg_attn_prefill": (C.c_int, [P, I32, I32, C.POINTER(AttnShape), P, P, P, I32, P, I32, P]),
+        "wg_prefill_layers": (C.c_int, [C.POINTER(PrefillLayer), I32, C.POINTER(PrefillBatch),
+                                        P]),
         "wg_attn_decode": (C.c_int, [P, I32, I32, C.POINTER(AttnShape), P, P, P, I32, P, I32,
                                      P, SZ, P]),
         "wg_attn_decode_prep": (C.c_int, [P, I32, I32, C.POINTER(AttnShape), P, P, P, I32, I32,

@@ -438,6 +438,12 @@ def attn_prefill(q: torch.Tensor, shape, k_cache, v_cache, pos0: torch.Tensor,
     return out
 
 
+def prefill_layers(layers, batch) -> None:
+    """A prompt batch through its layers in one call (wg_prefill_layers):
+    `layers` is an array of L.PrefillLayer, `batch` an L.PrefillBatch."""
+    L.check(L.load().wg_prefill_layers(layers, len(layers), C.byref(batch), _stream()))
+
+
 def short_conv(bcx, D, W, taps, state, state_out=None, prefixes=None, out=None):
     bcx = _dev(bcx, torch.float32)
     M = bcx.shape[0]
