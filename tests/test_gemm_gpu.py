@@ -117,7 +117,7 @@ def test_gemm_every_tile(hip, fmt, tile):
     assert e16 <= 1e-5
 
 
-@pytest.mark.parametrize("tile", [4, 5, 6, 7])
+@pytest.mark.parametrize("tile", [4, 5, 6, 7, 8])
 @pytest.mark.parametrize("fmt", ["q4_0", "nbits", "q4_k_rowgroup", "q8"])
 def test_gemm_wave_groups(hip, fmt, tile):
     """Each tile whose wave groups split K: one step (all groups but one
@@ -126,7 +126,7 @@ def test_gemm_wave_groups(hip, fmt, tile):
     from webgllm_amd import lib as L, ops
     L.tuning_set("gemm_tile", tile)
     try:
-        for M, N, K in ((1, 128, 256), (33, 384, 768), (70, 256, 2304)) + \
+        for M, N, K in ((1, 128, 256), (33, 384, 768), (150, 256, 2304)) + \
                 (() if fmt.startswith("q4_k") else ((65, 128, 64), (40, 128, 576))):
             m = _matrix(fmt, N, K, seed=tile + K)
             e, e16 = _check(m, M, seed=M, residual=K == 768)

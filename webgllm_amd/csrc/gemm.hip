@@ -774,7 +774,7 @@ int launch(const wg_q4_matrix *w, const uint16_t *A, int M, int lda, float *C, i
   const int cus = persistent_grid(1 << 30, 1);
   int t = tuning("gemm_tile");
   // Wave groups (4: 64 x 128 and 2 groups, 5: 64 x 64 and 4, 6: 32 x 32 and
-  // 8, 7: 32 x 64 and 4): the smallest tile whose workgroups all run at once
+  // 8, 7: 32 x 64 and 4, 8: 128 x 128 and 2): the smallest tile whose workgroups all run at once
   // (7's rings leave room for two a compute unit but for 8-bit weights), so
   // that no weight waits for a second round and no sum goes through memory.
   // Microseconds, with groups / the forms below: 131 rows of 896 -> 1152 6.8
@@ -795,10 +795,24 @@ int launch(const wg_q4_matrix *w, const uint16_t *A, int M, int lda, float *C, i
     else if (shallow && m64 * (w->N / 64) <= cus) t = 5;
     else if (shallow && w->N % 128 == 0 && m64 * (w->N / 128) <= cus) t = 4;
   }
-  if (t == 0) {
+  // 128 x 128 tiles that run at most one a compute unit leave its SIMDs a
+  // wave each: two wave groups a tile (8), or up to 2048 deep, where the
+  // groups' own loops are short, the smaller tiles. Microseconds, 128 x 128
+  // / this: 100 rows of 4096 -> 28672 57.2 (64 x 128) / 44.5 (8), 512 of
+  // 4096 -> 6144 60.4 / 55.5 (8), 1500 of 8192 -> 2048 85.0 / 78.5 (8), 1500
+  // of 2048 -> 2048 42.6 / 32.0 (64 x 128), 512 of 2048 -> 8192 43.4 / 33.3
+  // (64 x 128). Below 512 rows only half zero points, whose dequant costs
+  // most, pay for the taller tile (200 rows of 4096 -> 14336, Q4_0: 46.4 on
+  // 64 x 128 against 50.9). Past 8192 deep 128 rows pay from 257 on (300 of 14336 ->
+  // 4096: 87.9 against 100.4 on 64 x 128; 192: 65.5 against 60.4).
+  if (t == 0 && w->N % 128 == 0) {
+    const int64_t t2 = (int64_t)((M + 127) / 128) * (w->N / 128);
+    const int K = w->K;
     if (w->N % 256 == 0 && (int64_t)((M + 127) / 128) * (w->N / 256) * 4 >= (int64_t)cus * 3) t = 3;
-    else if (M >= 512 && w->N % 128 == 0) t = 2;
-    else if (w->N % 128 == 0) t = 1;
+    else if (K >= 768 && K <= 2048 && t2 <= cus) t = 1;
+    else if (K > 2048 && K <= 8192 && t2 <= cus && 4 * t2 >= 3 * cus &&
+             (M >= 512 || ZK == WG_ZERO_F16) && tuning("gemm_splits") <= 1) t = 8;
+    else t = M >= (K > 8192 ? 257 : 512) ? 2 : 1;
   }
 #define WG_GROUPS(BM, BN, S, WN, KG) \
   launch_groups<ZK, BM, BN, S, 1, WN, KG, SW>(w, A, M, lda, C, ldc, residual, ldr, row_scale, col_of, s)
@@ -806,6 +820,7 @@ int launch(const wg_q4_matrix *w, const uint16_t *A, int M, int lda, float *C, i
   if (t == 5) return WG_GROUPS(64, 64, 3, 2, 4);
   if (t == 6) return WG_GROUPS(32, 32, 3, 1, 8);
   if (t == 7) return WG_GROUPS(32, 64, 3, 2, 4);
+  if (t == 8 && w->N % 128 == 0) return WG_GROUPS(128, 128, ZK == Q8 ? 2 : 3, 4, 2);
 #undef WG_GROUPS
   if (t == 3 && w->N % 256 == 0) {
     if (tuning("gemm_pingpong"))
