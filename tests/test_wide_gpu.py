@@ -205,3 +205,23 @@ def test_embed_wide(hip, fmt):
     dense = _oracle_of(m).dense()
     assert np.array_equal(h[:3], dense[ids[:3]])
     assert not h[3:].any()
+
+
+@pytest.mark.parametrize("fmt,N", [("q8", 65536), ("q8", 65532), ("q6_k", 98304), ("q6_k", 98300)])
+def test_workgroups_a_cu_keep_the_bits(hip, fmt, N):
+    """A vocabulary's row groups on more workgroups a compute unit (on and
+    just under the line): the bits of 2 a unit."""
+    from webgllm_amd import lib as L, ops
+    K = 256
+    rng = np.random.default_rng(N)
+    m = ops.Q4Matrix.from_q8_0(_t(_q8_0_bytes(rng, N, K)), N, K) if fmt == "q8" else \
+        ops.Q4Matrix.from_q6_k(_t(_q6_k_bytes(rng, N, K)), N, K)
+    x = torch.randn((1, K), device="cuda").half()
+    got = ops.gemv(m, x)
+    old = L.tuning_get("wide_wg_per_cu")
+    L.tuning_set("wide_wg_per_cu", 2)
+    try:
+        want = ops.gemv(m, x)
+    finally:
+        L.tuning_set("wide_wg_per_cu", old)
+    assert torch.equal(got, want)

@@ -49,6 +49,7 @@ __device__ inline uint32_t comp(const uint4 &v, int c) {
 }
 
 struct Q8 {
+  static int per_cu(int G) { return G >= 16384 ? 8 : 2; }
   static constexpr int AV = 4;    // uint4 activation loads a chunk takes per token
   static constexpr int NSUM = 1;  // activation sums a chunk needs per token
   template <int NB>
@@ -127,6 +128,7 @@ struct Q8 {
 };
 
 struct Q6K {
+  static int per_cu(int G) { return G >= 24576 ? 4 : 2; }
   static constexpr int AV = 8;
   static constexpr int NSUM = 4;
   template <int NB>
@@ -363,7 +365,14 @@ template <class F, int M, int NB, int KS>
 int launch_stream(const Mat &mat, int G, const uint16_t *x, int ldx, float *y, int ldy,
                   const wg_epilogue &e, hipStream_t s) {
   constexpr int RGW = 4 / KS;
-  int grid = persistent_grid((G + RGW - 1) / RGW, tuning("wide_wg_per_cu"));
+  // Workgroups a compute unit: the knob, or 2, and more for a vocabulary's
+  // row groups, whose many rounds a slow workgroup would hold up (us at 2 /
+  // 4 / 8, one row: Q6_K 128256 x 4096 83.2 / 79.1 / 80.3, 65536 x 2048 31.3 /
+  // 32.4 / 34.0, 20000 x 4096 18.5 / 19.8 / 21.8; 8-bit 128256 x 4096 99.1 /
+  // 95.0 / 93.3, 65536 x 2048 28.6 / 27.6 / 27.4, 16384 x 2048 9.8 at each).
+  int per_cu = tuning("wide_wg_per_cu");
+  if (!per_cu) per_cu = M == 1 ? F::per_cu(G) : 2;  // (two rows: equal or slower)
+  int grid = persistent_grid((G + RGW - 1) / RGW, per_cu);
   if (e.mode == WG_EPI_SWIGLU)
     gemv_wide_stream_kernel<F, M, NB, KS, WG_EPI_SWIGLU><<<grid, 256, 0, s>>>(mat, x, ldx, y, ldy,
                                                                              e, G);
