@@ -143,6 +143,18 @@ def test_gemm_wave_groups(hip, fmt, tile):
         L.tuning_set("gemm_tile", 0)
 
 
+@pytest.mark.parametrize("fmt,M,N,K", [
+    ("q4_0", 33, 512, 768), ("q4_0", 300, 1024, 768), ("q8", 300, 2048, 768),
+    ("nbits", 200, 8192, 768), ("q4_0", 600, 6144, 2304), ("q4_0", 520, 4096, 1024),
+    ("q4_0", 257, 1024, 8448), ("nbits", 256, 1024, 8448)])
+def test_gemm_chosen_tiles(hip, fmt, M, N, K):
+    """The rule's own choice on both sides of its lines: each wave-group tile,
+    128 x 128 in two groups, 64 x 128 where 2048 deep or less, 128 rows past
+    8192 deep."""
+    e, e16 = _check(_matrix(fmt, N, K, seed=M), M, seed=K)
+    assert e <= 1e-3 and e16 <= 1e-5
+
+
 def test_gemm_column_map(hip):
     """col_of sends stored row n to output column col_of[n]: the mapped
     product equals the plain one with its columns permuted (bit for bit);
