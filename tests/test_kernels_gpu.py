@@ -511,3 +511,21 @@ def test_argmax_advance(hip, V):
     # no history
     ops.argmax_advance(_t(x), ids, pos)
     assert pos.item() == 9
+
+
+@pytest.mark.parametrize("D", [4, 1020, 1024, 1028, 4096, 4100, 8192, 8196])
+def test_norm_to_h2_rows(hip, D):
+    """The prescaled norm on both sides of each held row length: half(x w / 32)
+    bit for bit (one float32 product, an exact scaling, one rounding to half),
+    the row scale within float32 summation of the squares."""
+    from webgllm_amd import ops
+    rng = np.random.default_rng(D)
+    x = rng.standard_normal((5, D)).astype(np.float32)
+    w = rng.uniform(0.5, 1.5, D).astype(np.float32)
+    out = torch.empty((5, D), dtype=torch.float16, device="cuda")
+    rs = torch.empty(5, device="cuda")
+    ops.norm_to_h2(_t(x), _t(w), 1e-5, out, rs)
+    want = ((x * w).astype(np.float32) / np.float32(32)).astype(np.float16)
+    assert np.array_equal(out.cpu().numpy().view(np.uint16), want.view(np.uint16))
+    exact = 32 / np.sqrt((x.astype(np.float64) ** 2).mean(1) + 1e-5)
+    assert np.allclose(rs.cpu().numpy(), exact, rtol=2e-6)
