@@ -266,15 +266,15 @@ def test_gemm_split_k_first_launches(hip):
 
 
 def test_gemm_split_k_prefill_shape_in_graph(hip):
-    """The 512 x 4096 -> 4096 prefill GEMM (split by default when eager)
+    """A 512 x 14336 -> 4096 prefill GEMM (split 4 ways by default when eager)
     captured in a graph runs unsplit: every replay equals the unsplit result
     bit for bit, also with eager split launches on the capture stream
     between replays and after the stream's workspace has grown, and when
     replayed on another stream; the eager launches equal one another."""
     from webgllm_amd import lib as L, ops
-    m = _matrix("nbits", 4096, 4096, seed=5)
+    m = _matrix("nbits", 4096, 14336, seed=5)
     rng = np.random.default_rng(5)
-    a = _t(O.f32_to_h2(rng.standard_normal((512, 4096)).astype(np.float32)).view(np.int16))
+    a = _t(O.f32_to_h2(rng.standard_normal((512, 14336)).astype(np.float32)).view(np.int16))
     L.tuning_set("gemm_splits", 1)
     try:
         unsplit = ops.gemm(m, a)
@@ -285,6 +285,7 @@ def test_gemm_split_k_prefill_shape_in_graph(hip):
     with torch.cuda.stream(s):
         eager = ops.gemm(m, a)  # this stream's workspace
         torch.cuda.synchronize()
+        assert not torch.equal(eager, unsplit)  # (it does split)
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g, stream=s):
             ops.gemm(m, a, out=out)
@@ -295,15 +296,15 @@ def test_gemm_split_k_prefill_shape_in_graph(hip):
             torch.cuda.synchronize()
             assert torch.equal(out, unsplit), i
             assert torch.equal(other, eager), i
-        # a 4-way split needs more room: the workspace grows (is freed and
+        # an 8-way split needs more room: the workspace grows (is freed and
         # allocated again)
-        L.tuning_set("gemm_splits", 4)
+        L.tuning_set("gemm_splits", 8)
         try:
-            four = ops.gemm(m, a)
+            eight = ops.gemm(m, a)
         finally:
             L.tuning_set("gemm_splits", 0)
         torch.cuda.synchronize()
-        assert rel_l2(four.cpu().numpy(), unsplit.cpu().numpy()) <= 1e-6
+        assert rel_l2(eight.cpu().numpy(), unsplit.cpu().numpy()) <= 1e-6
     out.fill_(float("nan"))
     g.replay()  # on the current stream, not the capture stream
     torch.cuda.synchronize()
