@@ -47,7 +47,11 @@ const char *wg_version(void);
  * GEMV workgroups per compute unit) and
  * "gemv_min_waves" (below this many waves a GEMV splits K inside a
  * workgroup) and "gemm_tile" (prefill GEMM tile: 1 64 x 128, 2 128 x 128,
- * 3 128 x 256, or 0 to choose by shape) and "gemm_pingpong" (its 128 x 256
+ * 3 128 x 256; groups of waves that split K inside a workgroup: 4 64 x 128,
+ * 5 64 x 64, 6 32 x 32, 7 32 x 64, 8 128 x 128; or 0 to choose by shape),
+ * "gemm_splits" (K split that many ways between workgroups: 2, 4 or 8; 1
+ * splits it neither between workgroups nor between waves; 0 chooses) and
+ * "gemm_pingpong" (the 128 x 256
  * tiles with two wave groups half a K step apart, 1, or in lock-step, 0,
  * the default: the lock-step form runs two workgroups a compute unit).
  * Process-wide; results never depend on them. */

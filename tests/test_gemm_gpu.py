@@ -155,6 +155,30 @@ def test_gemm_chosen_tiles(hip, fmt, M, N, K):
     assert e <= 1e-3 and e16 <= 1e-5
 
 
+@pytest.mark.parametrize("fmt", ["q4_0", "nbits", "q4_k_rowgroup", "q8"])
+@pytest.mark.parametrize("M,N,K", [(45, 1024, 2048), (300, 1024, 768), (200, 8192, 1024),
+                                   (600, 6144, 2304)])
+def test_gemm_unsplit_takes_no_wave_groups(hip, fmt, M, N, K):
+    """gemm_splits = 1, the self-check's plainest form, sums K in one wave's
+    order: the bits of the 64 x 128 tile unsplit, on shapes that the rule
+    gives to 8, 4, 2 and (128 rows) 2 wave groups."""
+    from webgllm_amd import lib as L, ops
+    m = _matrix(fmt, N, K, seed=M)
+    a = torch.randn((M, K), device="cuda").half()
+    chosen = ops.gemm(m, a)
+    L.tuning_set("gemm_splits", 1)
+    try:
+        plain = ops.gemm(m, a)
+        L.tuning_set("gemm_tile", 1)
+        want = ops.gemm(m, a)
+    finally:
+        L.tuning_set("gemm_tile", 0)
+        L.tuning_set("gemm_splits", 0)
+    assert torch.equal(plain, want)
+    assert not torch.equal(plain, chosen)  # (the rule does take groups here)
+    assert rel_l2(plain.cpu().numpy(), chosen.cpu().numpy()) <= 1e-6
+
+
 def test_gemm_column_map(hip):
     """col_of sends stored row n to output column col_of[n]: the mapped
     product equals the plain one with its columns permuted (bit for bit);

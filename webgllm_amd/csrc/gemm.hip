@@ -56,6 +56,7 @@
 #include "common.h"
 #include "dot.h"
 #include "gemm_core.h"
+#include "gemm_rule.h"
 #include "kernels.h"
 #include "lds_load.h"
 
@@ -737,13 +738,9 @@ int launch_tiles(const wg_q4_matrix *w, const uint16_t *A, int M, int lda, float
   // to 4) while the workgroups stay within two a compute unit (one for the
   // 8-wave tile) and every split keeps at least S steps.
   int ks = tuning("gemm_splits");
-  if (ks == 0) {
-    const int64_t room = (int64_t)persistent_grid(1 << 30, 1) * (WGM * WGN > 4 ? 1 : 2);
-    ks = 1;
-    while (ks < 4 && (int64_t)tiles * ks * 2 <= room && steps % (2 * ks) == 0 &&
-           steps / (2 * ks) >= S)
-      ks *= 2;
-  }
+  if (ks == 0)
+    ks = gemm_k_splits(tiles, steps, S,
+                       (int64_t)persistent_grid(1 << 30, 1) * (WGM * WGN > 4 ? 1 : 2));
   // (the slots are read by 32-bit buffer offsets: under 2 GiB of them)
   if ((ks & (ks - 1)) || ks > 8 || steps % ks ||
       (int64_t)(2 * ks - 2) * tiles * BM * BN * 4 >= ((int64_t)1 << 31))
@@ -766,54 +763,12 @@ template <int ZK, bool SW = false>
 int launch(const wg_q4_matrix *w, const uint16_t *A, int M, int lda, float *C, int ldc,
            const float *residual, int ldr, const float *row_scale, const int32_t *col_of,
            hipStream_t s) {
-  // Each weight is dequantized once per tile, so taller tiles (more rows a
-  // wave) spend fewer vector instructions per MFMA: 128 x 256 where its
-  // tiles cover most compute units, else 128 x 128 from 512 rows, else 64 x
-  // 128; splitting K makes up the workgroups that few tiles leave short.
-  // The knob gemm_tile forces one (1: 64 x 128, 2: 128 x 128, 3: 128 x 256).
-  const int cus = persistent_grid(1 << 30, 1);
+  // The tile: the knob gemm_tile, or by sizes; wave groups only where the
+  // knob gemm_splits leaves the splitting of K to the rule (1 is the plainest
+  // form: every sum in one wave's order).
   int t = tuning("gemm_tile");
-  // Wave groups (4: 64 x 128 and 2 groups, 5: 64 x 64 and 4, 6: 32 x 32 and
-  // 8, 7: 32 x 64 and 4, 8: 128 x 128 and 2): the smallest tile whose workgroups all run at once
-  // (7's rings leave room for two a compute unit but for 8-bit weights), so
-  // that no weight waits for a second round and no sum goes through memory.
-  // Microseconds, with groups / the forms below: 131 rows of 896 -> 1152 6.8
-  // / 12.5 (6), 896 -> 9728 10.7 / 15.0 (4), 4864 -> 896 12.4 / 23.9 (6); 45
-  // rows, 8-bit, 2048 -> 16384 13.6 / 20.2 (5), 8192 -> 2048 15.8 / 23.0
-  // (6); 512 rows of 2048 -> 2048 13.4 / 28.8 (7), 4096 -> 4096 40.7 / 51.4
-  // (4). Past those workgroups they are slower (512 rows of 896 -> 9728 28.9
-  // / 22.7), and past 8192 deep, where the loop outweighs the splits'
-  // meeting, no faster (131 rows of 14336 -> 4096 63 / 60; 6, with 45 rows,
-  // 32.9 / 45.0). Rows under 768 deep (12 steps) keep the forms below too:
-  // the groups would save them 4 of 8 to 10 us, but models that narrow are
-  // tests', whose greedy picks follow the order of the sums.
-  if (t == 0 && w->K >= 768 && tuning("gemm_splits") <= 1) {  // (2 and more force splits)
-    const int64_t m32 = (M + 31) / 32, m64 = (M + 63) / 64;
-    const bool shallow = w->K <= 8192;
-    if (m32 * (w->N / 32) <= cus) t = 6;
-    else if (shallow && m32 * (w->N / 64) <= (ZK == Q8 ? 1 : 2) * cus) t = 7;
-    else if (shallow && m64 * (w->N / 64) <= cus) t = 5;
-    else if (shallow && w->N % 128 == 0 && m64 * (w->N / 128) <= cus) t = 4;
-  }
-  // 128 x 128 tiles that run at most one a compute unit leave its SIMDs a
-  // wave each: two wave groups a tile (8), or up to 2048 deep, where the
-  // groups' own loops are short, the smaller tiles. Microseconds, 128 x 128
-  // / this: 100 rows of 4096 -> 28672 57.2 (64 x 128) / 44.5 (8), 512 of
-  // 4096 -> 6144 60.4 / 55.5 (8), 1500 of 8192 -> 2048 85.0 / 78.5 (8), 1500
-  // of 2048 -> 2048 42.6 / 32.0 (64 x 128), 512 of 2048 -> 8192 43.4 / 33.3
-  // (64 x 128). Below 512 rows only half zero points, whose dequant costs
-  // most, pay for the taller tile (200 rows of 4096 -> 14336, Q4_0: 46.4 on
-  // 64 x 128 against 50.9). Past 8192 deep 128 rows pay from 257 on (300 of 14336 ->
-  // 4096: 87.9 against 100.4 on 64 x 128; 192: 65.5 against 60.4).
-  if (t == 0 && w->N % 128 == 0) {
-    const int64_t t2 = (int64_t)((M + 127) / 128) * (w->N / 128);
-    const int K = w->K;
-    if (w->N % 256 == 0 && (int64_t)((M + 127) / 128) * (w->N / 256) * 4 >= (int64_t)cus * 3) t = 3;
-    else if (K >= 768 && K <= 2048 && t2 <= cus) t = 1;
-    else if (K > 2048 && K <= 8192 && t2 <= cus && 4 * t2 >= 3 * cus &&
-             (M >= 512 || ZK == WG_ZERO_F16) && tuning("gemm_splits") <= 1) t = 8;
-    else t = M >= (K > 8192 ? 257 : 512) ? 2 : 1;
-  }
+  if (t == 0)
+    t = gemm_tile_for(ZK, M, w->N, w->K, persistent_grid(1 << 30, 1), tuning("gemm_splits") == 0);
 #define WG_GROUPS(BM, BN, S, WN, KG) \
   launch_groups<ZK, BM, BN, S, 1, WN, KG, SW>(w, A, M, lda, C, ldc, residual, ldr, row_scale, col_of, s)
   if (t == 4 && w->N % 128 == 0) return WG_GROUPS(64, 128, 4, 4, 2);
