@@ -475,12 +475,12 @@ int wg_q4_gemv(const wg_q4_matrix *w, const uint16_t *x, int32_t M, int32_t ldx,
  * order (the loaders' srcRows, stored row n = logical row col_of[n]) then
  * comes out in logical order; entries outside 0..N-1 are not written.
  * Short prompts and small matrices split K between the waves of a workgroup,
- * whose sums meet in LDS in a fixed order, captured or not. Elsewhere, where
- * tiles are fewer than the compute units, K is split 2 or 4 ways and
- * the partial sums are added in a fixed pairwise order (bits independent of
- * which split ends last), in a workspace the library keeps per stream and
- * grows on demand; launches on one stream run in turn. A launch made while
- * its stream is being captured into a graph runs unsplit (the graph holds
+ * whose sums meet in LDS in a fixed order. Elsewhere, where tiles are fewer
+ * than the compute units, K is split 2 or 4 ways and the partial sums are
+ * added in a fixed pairwise order (bits independent of which split ends
+ * last), in a workspace the library keeps per stream and grows on demand;
+ * launches on one stream run in turn. A launch made while its stream is
+ * being captured into a graph takes the first form or none (the graph holds
  * no workspace, so it may replay on any stream and beside eager GEMMs), and
  * so its sums may differ in the last bits from an eager launch's.
  * A WG_ZERO_Q4K matrix's (d', z') halves are rebuilt first, bit for bit as

@@ -22,8 +22,9 @@ def rule(tmp_path_factory):
     d = tmp_path_factory.mktemp("rule")
     src, so = d / "rule.cpp", d / "rule.so"
     src.write_text(f'#include "{CSRC}/gemm_rule.h"\n'
-                   'extern "C" int tile(int zk, int M, int N, int K, int cus, int groups) {\n'
-                   '  return wg::gemm_tile_for(zk, M, N, K, cus, groups != 0);\n}\n')
+                   'extern "C" int tile(int zk, int M, int N, int K, int cus, int groups,'
+                   ' int splits) {\n'
+                   '  return wg::gemm_tile_for(zk, M, N, K, cus, groups != 0, splits != 0);\n}\n')
     subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-o",
                     str(so), str(src)], check=True)
     return C.CDLL(str(so))
@@ -35,5 +36,36 @@ def test_plain_settings_take_no_wave_groups(rule):
     assert PLAIN_TUNING["gemm_splits"] == 1
     for zk in ZK.values():
         for M, N, K in SIZES:
-            assert rule.tile(zk, M, N, K, CUS, 0) <= 3, (zk, M, N, K)
-    assert any(rule.tile(0, M, N, K, CUS, 1) >= 4 for M, N, K in SIZES)
+            assert rule.tile(zk, M, N, K, CUS, 0, 0) <= 3, (zk, M, N, K)
+    assert any(rule.tile(0, M, N, K, CUS, 1, 1) >= 4 for M, N, K in SIZES)
+
+
+# (form, M, N, K, the tile where splits may run, the tile under capture): each
+# a shape that another tile had taken 5 to 44% longer for
+@pytest.mark.parametrize("zk,M,N,K,tile,captured", [
+    # one 64 x 64 a compute unit, not two 32 x 64
+    ("f16", 300, 2048, 8192, 5, 5), ("q4_0", 33, 9728, 8192, 5, 5), ("u8", 45, 9728, 4864, 5, 5),
+    ("u8", 33, 9728, 8192, 1, 5), ("q4_0", 131, 6144, 8192, 7, 7), ("q4_0", 700, 896, 768, 7, 7),
+    # 64 x 128 in two groups only while the splits of one are slower
+    ("q4_0", 100, 9728, 8192, 1, 4), ("q4_0", 1024, 1152, 8192, 1, 4),
+    ("u8", 300, 4096, 8192, 1, 4), ("u8", 300, 4096, 4096, 4, 4),
+    ("f16", 1500, 896, 8192, 2, 4), ("f16", 131, 9728, 8192, 4, 4),
+    ("q8", 1024, 1152, 8192, 2, 4), ("q8", 131, 6144, 8192, 7, 7),
+    # half zero points' 64 x 128 to 1536 deep
+    ("f16", 2048, 2048, 2048, 2, 2), ("q4_0", 2048, 2048, 2048, 1, 1),
+    # 128 rows past 8192 deep: a split more, a costly dequant
+    ("f16", 300, 4096, 14336, 2, 1), ("q8", 300, 4096, 14336, 2, 1),
+    ("f16", 300, 9728, 8448, 2, 2), ("q4_0", 300, 4096, 14336, 1, 1), ("q8", 257, 6144, 8448, 1, 1),
+    ("f16", 300, 1152, 14336, 1, 1), ("q4_0", 400, 1152, 8448, 1, 1)])
+def test_lines(rule, zk, M, N, K, tile, captured):
+    assert rule.tile(ZK[zk], M, N, K, CUS, 1, 1) == tile
+    assert rule.tile(ZK[zk], M, N, K, CUS, 1, 0) == captured
+
+
+def test_tiles_divide_the_columns(rule):
+    """Every tile's columns divide N (a multiple of 64)."""
+    cols = {0: 64, 1: 128, 2: 128, 3: 256, 4: 128, 5: 64, 6: 32, 7: 64, 8: 128}
+    for zk in ZK.values():
+        for M, N, K in SIZES + [(M, N + 64, K) for M, N, K in SIZES]:
+            for groups, splits in ((1, 1), (1, 0), (0, 0)):
+                assert N % cols[rule.tile(zk, M, N, K, CUS, groups, splits)] == 0

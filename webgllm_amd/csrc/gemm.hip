@@ -594,6 +594,16 @@ struct SplitSpace {
   int counters;
 };
 
+// Whether s is being captured (or a capture elsewhere forbids asking).
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return cs != hipStreamCaptureStatusNone;
+}
+
 // The workspace for `floats` partial floats and `counters` counters on
 // stream s; part stays null while s is being captured into a graph (the
 // launch runs unsplit).
@@ -602,12 +612,7 @@ int split_space(hipStream_t s, size_t floats, int counters, float **part, int **
   static std::vector<SplitSpace *> spaces;
   *part = nullptr;
   *count = nullptr;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
-    (void)hipGetLastError();
-    return WG_OK;
-  }
-  if (cs != hipStreamCaptureStatusNone) return WG_OK;
+  if (capturing(s)) return WG_OK;
   int dev = 0;
   WG_HIP(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lock(mu);
@@ -667,12 +672,7 @@ int expand_space(hipStream_t s, size_t count, uint16_t **out) {
   static std::mutex mu;
   static std::vector<ExpandSpace *> spaces;
   *out = nullptr;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
-    (void)hipGetLastError();
-    return WG_OK;
-  }
-  if (cs != hipStreamCaptureStatusNone) return WG_OK;
+  if (capturing(s)) return WG_OK;
   int dev = 0;
   WG_HIP(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lock(mu);
@@ -767,8 +767,13 @@ int launch(const wg_q4_matrix *w, const uint16_t *A, int M, int lda, float *C, i
   // knob gemm_splits leaves the splitting of K to the rule (1 is the plainest
   // form: every sum in one wave's order).
   int t = tuning("gemm_tile");
-  if (t == 0)
-    t = gemm_tile_for(ZK, M, w->N, w->K, persistent_grid(1 << 30, 1), tuning("gemm_splits") == 0);
+  if (t == 0) {
+    const int cus = persistent_grid(1 << 30, 1);
+    const bool groups = tuning("gemm_splits") == 0;
+    t = gemm_tile_for(ZK, M, w->N, w->K, cus, groups, groups);
+    const int whole = gemm_tile_for(ZK, M, w->N, w->K, cus, groups, false);
+    if (t != whole && capturing(s)) t = whole;
+  }
 #define WG_GROUPS(BM, BN, S, WN, KG) \
   launch_groups<ZK, BM, BN, S, 1, WN, KG, SW>(w, A, M, lda, C, ldc, residual, ldr, row_scale, col_of, s)
   if (t == 4 && w->N % 128 == 0) return WG_GROUPS(64, 128, 4, 4, 2);

@@ -21,51 +21,87 @@ inline int gemm_k_splits(int64_t tiles, int steps, int stages, int64_t room) {
 // The tile of an M x N x K product of weight form zk on `cus` compute units:
 // 0 64 x 64, 1 64 x 128, 2 128 x 128, 3 128 x 256; wave groups 4 64 x 128
 // (2 of them), 5 64 x 64 (4), 6 32 x 32 (8), 7 32 x 64 (4), 8 128 x 128 (2).
-// groups: whether wave groups may be taken.
-inline int gemm_tile_for(int zk, int M, int N, int K, int cus, bool groups) {
-  // The smallest tile whose workgroups all run at once (7's rings leave room
-  // for two a compute unit but for 8-bit weights), so that no weight waits
-  // for a second round and no sum goes through memory. Microseconds, with
-  // groups / the forms below: 131 rows of 896 -> 1152 6.8 / 12.5 (6), 896 ->
-  // 9728 10.7 / 15.0 (4), 4864 -> 896 12.4 / 23.9 (6); 45 rows, 8-bit, 2048
-  // -> 16384 13.6 / 20.2 (5), 8192 -> 2048 15.8 / 23.0 (6); 512 rows of 2048
-  // -> 2048 13.4 / 28.8 (7), 4096 -> 4096 40.7 / 51.4 (4). Past those
-  // workgroups they are slower (512 rows of 896 -> 9728 28.9 / 22.7), and
-  // past 8192 deep, where the loop outweighs the splits' meeting, no faster
-  // (131 rows of 14336 -> 4096 63 / 60; 6, with 45 rows, 32.9 / 45.0). Rows
-  // under 768 deep (12 steps) keep the forms below too: the groups would save
-  // them 4 of 8 to 10 us, but models that narrow are tests', whose greedy
-  // picks follow the order of the sums.
+// groups: whether wave groups may be taken; splits: whether 0 to 3 may split
+// K between workgroups (not while a stream is captured).
+//
+// Every line was measured on a grid of 9 to 2048 rows, 256 to 28672 columns
+// and 768 to 14336 deep, all four weight forms, eager launches over several
+// matrices; "/" stands between this tile and the one on the line's other side,
+// in microseconds.
+inline int gemm_tile_for(int zk, int M, int N, int K, int cus, bool groups, bool splits) {
+  const int64_t m32 = (M + 31) / 32, m64 = (M + 63) / 64, m128 = (M + 127) / 128;
+  // Wave groups: the smallest tile whose workgroups all run at once, so that
+  // no weight waits for a second round and no sum goes through memory (131
+  // rows of 896 -> 1152 6.8 / 12.5 (6), 4864 -> 896 12.4 / 23.9 (6); 45 rows,
+  // 8-bit, 2048 -> 16384 13.6 / 20.2 (5); 512 rows of 4096 -> 4096 25.5 /
+  // 31.7 (4)). Past those workgroups they are slower (512 rows of 896 -> 9728
+  // 28.9 / 22.7). Past 8192 deep, where the loop outweighs the splits'
+  // meeting, only 32 x 32 is faster (45 rows of 14336 -> 4096 32.9 / 45.0).
+  // Rows under 768 deep (12 steps) keep the forms below too: the groups would
+  // save them 4 of 8 to 10 us, but models that narrow are tests', whose
+  // greedy picks follow the order of the sums.
   if (groups && K >= 768) {
-    const int64_t m32 = (M + 31) / 32, m64 = (M + 63) / 64;
     const bool shallow = K <= 8192;
     if (m32 * (N / 32) <= cus) return 6;
-    if (shallow && m32 * (N / 64) <= (zk == Q8 ? 1 : 2) * cus) return 7;
-    if (shallow && m64 * (N / 64) <= cus) return 5;
-    if (shallow && N % 128 == 0 && m64 * (N / 128) <= cus) return 4;
+    if (shallow && m32 * (N / 64) <= cus) return 7;
+    // One 64 x 64 a compute unit against two 32 x 64: 300 rows of 4096 ->
+    // 3072, half zero points, 19.4 / 22.4, 400 of 8192 -> 2048, Q4_0, 26.1 /
+    // 29.5; under 1024 deep the two are as fast or faster (Q4_0 at 768 2% in
+    // the mean). Byte zero points past 6144 deep gain nothing on the split 64
+    // x 128 (33 rows of 8192 -> 9728 28.3 / 25.4).
+    if (shallow && m64 * (N / 64) <= cus && (zk == Q8 || K >= 1024)) {
+      if (splits && zk == WG_ZERO_U8 && K > 6144) return N % 128 ? 0 : 1;
+      return 5;
+    }
+    // Two 32 x 64 a compute unit (their rings leave room, an 8-bit one's but
+    // just: from 2048 deep): 131 rows of 4096 -> 6144 17.0 / 21.4, 8192 ->
+    // 6144 30.5 / 36.3.
+    if (shallow && m32 * (N / 64) <= 2 * cus && (zk != Q8 || K >= 2048)) return 7;
+    // 64 x 128 in two groups, up to where the splits of one group catch up:
+    // Q4_0 first, whose dequant is cheapest (100 rows of 8192 -> 9728 41.4 /
+    // 36.4), half zero points last and only at few rows (131 of 8192 -> 9728
+    // 56.0 / 58.7, 1500 of 8192 -> 896 55.9 / 46.6 on 128 x 128).
+    if (shallow && N % 128 == 0 && m64 * (N / 128) <= cus) {
+      const int deep = zk == WG_ZERO_8 ? 3072
+                       : zk == WG_ZERO_U8 ? 4096
+                       : zk == WG_ZERO_F16 ? (M < 512 ? 8192 : 4096) : (M < 512 ? 7168 : 6144);
+      if (!splits || K <= deep) return 4;
+      // (Q4_0, 1024 rows of 8192 -> 1152: 64 x 128 36.9, 128 x 128 39.8)
+      if (zk == WG_ZERO_8 || zk == WG_ZERO_U8) return 1;
+    }
   }
   if (N % 128) return 0;
   // Each weight is dequantized once per tile, so taller tiles (more rows a
   // wave) spend fewer vector instructions per MFMA: 128 x 256 where its
   // tiles cover most compute units, else 128 x 128 from 512 rows, else 64 x
   // 128; splitting K makes up the workgroups that few tiles leave short.
-  const int64_t m128 = (M + 127) / 128, t2 = m128 * (N / 128);
+  const int64_t t1 = m64 * (N / 128), t2 = m128 * (N / 128);
   if (N % 256 == 0 && m128 * (N / 256) * 4 >= (int64_t)cus * 3) return 3;
   // 128 x 128 tiles that run at most one a compute unit leave its SIMDs a
-  // wave each: two wave groups a tile (8), or up to 2048 deep, where the
-  // groups' own loops are short, the smaller tiles. Microseconds, 128 x 128
-  // / this: 100 rows of 4096 -> 28672 57.2 (64 x 128) / 44.5 (8), 512 of
-  // 4096 -> 6144 60.4 / 55.5 (8), 1500 of 8192 -> 2048 85.0 / 78.5 (8), 1500
-  // of 2048 -> 2048 42.6 / 32.0 (64 x 128), 512 of 2048 -> 8192 43.4 / 33.3
-  // (64 x 128). Below 512 rows only half zero points, whose dequant costs
-  // most, pay for the taller tile (200 rows of 4096 -> 14336, Q4_0: 46.4 on
-  // 64 x 128 against 50.9). Past 8192 deep 128 rows pay from 257 on (300 of 14336 ->
-  // 4096: 87.9 against 100.4 on 64 x 128; 192: 65.5 against 60.4).
-  if (K >= 768 && K <= 2048 && t2 <= cus) return 1;
+  // wave each: two wave groups a tile (8: 100 rows of 4096 -> 28672 44.5 /
+  // 57.2, 512 of 4096 -> 6144 55.5 / 60.4, 1500 of 8192 -> 2048 78.5 / 85.0),
+  // or up to 2048 deep, where the groups' own loops are short, 64 x 128
+  // (1500 of 2048 -> 2048 32.0 / 42.6, 512 of 2048 -> 8192 33.3 / 43.4, Q4_0;
+  // half zero points, whose dequant costs most, to 1536: 2048 of 2048 -> 1152
+  // 30.6 / 28.7). Below 512 rows only half zero points pay for 8 (200 rows
+  // of 4096 -> 14336, Q4_0: 50.9 / 46.4 on 64 x 128).
+  if (K >= 768 && K <= (zk == WG_ZERO_F16 ? 1536 : 2048) && t2 <= cus) return 1;
   if (groups && K > 2048 && K <= 8192 && t2 <= cus && 4 * t2 >= 3 * (int64_t)cus &&
       (M >= 512 || zk == WG_ZERO_F16))
     return 8;
-  return M >= (K > 8192 ? 257 : 512) ? 2 : 1;
+  // Past 8192 deep 128 rows pay below 512 where they alone leave room for
+  // another split, and only for the forms whose dequant costs most (300 rows
+  // of 14336 -> 4096: half zero points 72.2 / 93.4, 8-bit 67.3 / 74.1, byte
+  // zero points 63.9 / 65.5, Q4_0 61.9 / 59.9; -> 2048, both split 4 ways,
+  // 8-bit 49.4 / 44.5). Unsplit, half zero points pay where only 64 rows need
+  // a second round (300 of 8448 -> 9728 98.7 / 108.8).
+  if (K > 8192 && M > 256 && M < 512 && zk != WG_ZERO_8 && (zk != WG_ZERO_U8 || K > 11008)) {
+    const int64_t room = 2 * (int64_t)cus;
+    if (splits ? gemm_k_splits(t2, K / 64, 3, room) > gemm_k_splits(t1, K / 64, 4, room)
+               : zk == WG_ZERO_F16 && t1 > cus && t2 <= cus)
+      return 2;
+  }
+  return M >= 512 ? 2 : 1;
 }
 
 }  // namespace wg
