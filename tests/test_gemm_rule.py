@@ -41,7 +41,7 @@ def test_plain_settings_take_no_wave_groups(rule):
 
 
 # (form, M, N, K, the tile where splits may run, the tile under capture): each
-# a shape that another tile had taken 5 to 44% longer for
+# a shape beside a line, where the tile on its other side takes longer
 @pytest.mark.parametrize("zk,M,N,K,tile,captured", [
     # one 64 x 64 a compute unit, not two 32 x 64
     ("f16", 300, 2048, 8192, 5, 5), ("q4_0", 33, 9728, 8192, 5, 5), ("u8", 45, 9728, 4864, 5, 5),
@@ -51,6 +51,8 @@ def test_plain_settings_take_no_wave_groups(rule):
     ("u8", 300, 4096, 8192, 1, 4), ("u8", 300, 4096, 4096, 4, 4),
     ("f16", 1500, 896, 8192, 2, 4), ("f16", 131, 9728, 8192, 4, 4),
     ("q8", 1024, 1152, 8192, 2, 4), ("q8", 131, 6144, 8192, 7, 7),
+    # from 256 deep on
+    ("q4_0", 45, 1152, 256, 6, 6), ("q8", 300, 1536, 512, 7, 7), ("q4_0", 45, 1152, 192, 1, 1),
     # half zero points' 64 x 128 to 1536 deep
     ("f16", 2048, 2048, 2048, 2, 2), ("q4_0", 2048, 2048, 2048, 1, 1),
     # 128 rows past 8192 deep: a split more, a costly dequant

@@ -25,7 +25,7 @@ inline int gemm_k_splits(int64_t tiles, int steps, int stages, int64_t room) {
 // K between workgroups (not while a stream is captured).
 //
 // Every line was measured on a grid of 9 to 2048 rows, 256 to 28672 columns
-// and 768 to 14336 deep, all four weight forms, eager launches over several
+// and 64 to 14336 deep, all four weight forms, eager launches over several
 // matrices; "/" stands between this tile and the one on the line's other side,
 // in microseconds.
 inline int gemm_tile_for(int zk, int M, int N, int K, int cus, bool groups, bool splits) {
@@ -37,10 +37,9 @@ inline int gemm_tile_for(int zk, int M, int N, int K, int cus, bool groups, bool
   // 31.7 (4)). Past those workgroups they are slower (512 rows of 896 -> 9728
   // 28.9 / 22.7). Past 8192 deep, where the loop outweighs the splits'
   // meeting, only 32 x 32 is faster (45 rows of 14336 -> 4096 32.9 / 45.0).
-  // Rows under 768 deep (12 steps) keep the forms below too: the groups would
-  // save them 4 of 8 to 10 us, but models that narrow are tests', whose
-  // greedy picks follow the order of the sums.
-  if (groups && K >= 768) {
+  // Under 256 deep (4 steps) their groups have a step or none each (45 rows ->
+  // 1152, Q4_0: 64 deep 4.8 / 4.3, 256 deep 4.7 / 5.3, 512 deep 4.6 / 7.3).
+  if (groups && K >= 256) {
     const bool shallow = K <= 8192;
     if (m32 * (N / 32) <= cus) return 6;
     if (shallow && m32 * (N / 64) <= cus) return 7;
@@ -85,7 +84,7 @@ inline int gemm_tile_for(int zk, int M, int N, int K, int cus, bool groups, bool
   // half zero points, whose dequant costs most, to 1536: 2048 of 2048 -> 1152
   // 30.6 / 28.7). Below 512 rows only half zero points pay for 8 (200 rows
   // of 4096 -> 14336, Q4_0: 50.9 / 46.4 on 64 x 128).
-  if (K >= 768 && K <= (zk == WG_ZERO_F16 ? 1536 : 2048) && t2 <= cus) return 1;
+  if (K >= 256 && K <= (zk == WG_ZERO_F16 ? 1536 : 2048) && t2 <= cus) return 1;
   if (groups && K > 2048 && K <= 8192 && t2 <= cus && 4 * t2 >= 3 * (int64_t)cus &&
       (M >= 512 || zk == WG_ZERO_F16))
     return 8;
