@@ -143,16 +143,27 @@ def test_gemm_wave_groups(hip, fmt, tile):
         L.tuning_set("gemm_tile", 0)
 
 
-@pytest.mark.parametrize("fmt,M,N,K", [
-    ("q4_0", 33, 512, 768), ("q4_0", 300, 1024, 768), ("q8", 300, 2048, 768),
-    ("nbits", 200, 8192, 768), ("q4_0", 600, 6144, 2304), ("q4_0", 520, 4096, 1024),
-    ("q4_0", 257, 1024, 8448), ("nbits", 256, 1024, 8448)])
-def test_gemm_chosen_tiles(hip, fmt, M, N, K):
-    """The rule's own choice on both sides of its lines: each wave-group tile,
-    128 x 128 in two groups, 64 x 128 where 2048 deep or less, 128 rows past
-    8192 deep."""
-    e, e16 = _check(_matrix(fmt, N, K, seed=M), M, seed=K)
+@pytest.mark.parametrize("fmt,M,N,K,tile,other", [
+    ("q4_0", 33, 512, 768, 6, 7), ("q4_0", 300, 1024, 768, 7, 6), ("q8", 300, 2048, 768, 5, 4),
+    ("nbits", 200, 8192, 768, 4, 5), ("q4_0", 600, 6144, 2304, 8, 1),
+    ("q4_k_rowgroup", 200, 14336, 2304, 8, 1), ("q4_0", 520, 4096, 1024, 1, 8),
+    ("q8", 300, 4096, 8448, 2, 1), ("nbits", 256, 2048, 8448, 1, 6)])
+def test_gemm_chosen_tiles(hip, fmt, M, N, K, tile, other):
+    """The rule's own choice beside its lines (test_gemm_rule.py holds every
+    line): the product, and the bits of that tile forced, which another
+    tile's sums, in another order, do not give."""
+    from webgllm_amd import lib as L, ops
+    m = _matrix(fmt, N, K, seed=M)
+    e, e16 = _check(m, M, seed=K)
     assert e <= 1e-3 and e16 <= 1e-5
+    a = torch.randn((M, K), device="cuda").half()
+    chosen = ops.gemm(m, a)
+    try:
+        for t in (tile, other):
+            L.tuning_set("gemm_tile", t)
+            assert torch.equal(ops.gemm(m, a), chosen) == (t == tile), t
+    finally:
+        L.tuning_set("gemm_tile", 0)
 
 
 @pytest.mark.parametrize("fmt", ["q4_0", "nbits", "q4_k_rowgroup", "q8"])
