@@ -150,11 +150,11 @@ def test_delta_conv_matches_oracle(hip, M, C, W):
         assert np.array_equal(st_out.cpu().numpy()[:W - 1], want_state)
 
 
-@pytest.mark.parametrize("M", [8, 9, 15, 301])
-@pytest.mark.parametrize("C,W", [(4, 2), (1028, 3), (1024, 4)])
+@pytest.mark.parametrize("M,C,W", [(8, 50000, 2), (9, 44448, 3), (15, 26668, 4), (301, 1332, 3),
+                                   (391, 1024, 4), (390, 1024, 4), (100000, 4, 2)])
 def test_delta_conv_rows_equal_the_general_kernel(hip, M, C, W):
-    """Batches whose strides and arrays allow 16-byte loads run 8 rows a
-    thread: the outputs and states of the thread-an-output kernel (rows one
+    """Batches of 400,000 outputs or more (and one just under) whose strides
+    and arrays allow 16-byte loads run 8 rows a thread: the outputs and states of the thread-an-output kernel (rows one
     float further apart) bit for bit, the state from rows of the batch or,
     where it is short, of the old state."""
     from webgllm_amd import ops

@@ -207,6 +207,11 @@ __global__ __launch_bounds__(256) void delta_conv_kernel(const float *in, int ld
 // a thread an output, 16 us now (4.6 TB/s). Channels and strides are multiples of 4,
 // the arrays 16-byte aligned.
 constexpr int CONV_ROWS = 8;
+// Fewer outputs wait on memory round trips, which 32 times the threads hide
+// better (a graph of them, us, a thread an output / 8 rows of 4: 24 rows of
+// 6144 3.5 / 4.9, 41 3.9 / 4.6, 65 4.55 / 4.57, 98 5.7 / 4.7; 146 of 1024
+// 3.4 / 4.4, 391 4.6 / 4.6, 781 6.7 / 4.8).
+constexpr int CONV_ROWS_MIN = 400000;
 
 template <int W>
 __global__ __launch_bounds__(256) void delta_conv_rows_kernel(const float *in, int ldi, int M,
@@ -760,8 +765,9 @@ int wg_delta_conv(const float *in, int32_t M, int32_t ldi, int32_t C, int32_t W,
   WG_REQUIRE(W == 1 || (state && state_out && !overlaps(state, sb, state_out, sb)),
              "wg_delta_conv: %d taps need a state and a separate state_out", W);
   const uintptr_t ptrs = (uintptr_t)in | (uintptr_t)out | (uintptr_t)state | (uintptr_t)state_out;
-  if (M >= CONV_ROWS && W >= 2 && W <= 4 && C % 4 == 0 && ldi % 4 == 0 && ldo % 4 == 0 &&
-      (ptrs & 15) == 0 && (M + CONV_ROWS - 1) / CONV_ROWS <= 65535) {
+  if (M >= CONV_ROWS && (int64_t)M * C >= CONV_ROWS_MIN && W >= 2 && W <= 4 && C % 4 == 0 &&
+      ldi % 4 == 0 && ldo % 4 == 0 && (ptrs & 15) == 0 &&
+      (M + CONV_ROWS - 1) / CONV_ROWS <= 65535) {
     auto kernel = W == 2 ? delta_conv_rows_kernel<2>
                          : W == 3 ? delta_conv_rows_kernel<3> : delta_conv_rows_kernel<4>;
     kernel<<<dim3((C / 4 + 255) / 256, (M + CONV_ROWS - 1) / CONV_ROWS), 256, 0,
