@@ -177,6 +177,36 @@ def test_delta_chunked_at_tile_edges(hip, H, dk, dv, M, save_at):
     test_delta_chunked_matches_oracle(hip, H, dk, dv, M, save_at)
 
 
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("row", [0, 3, 14, 15, 16, 37, 63, 64, 90])
+@pytest.mark.parametrize("what", ["q", "k", "v", "beta", "decay"])
+def test_delta_chunked_keeps_earlier_rows(hip, what, row, bad):
+    """A value that is not finite reaches its own row and later ones alone:
+    every row before it, and every row of the other head, has the bits of a
+    clean batch (one row at a time no earlier row depends on it)."""
+    from webgllm_amd import ops
+    H, dk, dv, M = 2, 36, 40, 100
+    g = torch.Generator(device="cuda")
+    g.manual_seed(row)
+    qkv = torch.randn((M, 2 * H * dk + H * dv), device="cuda", generator=g)
+    ba = torch.randn((M, 2 * H), device="cuda", generator=g)
+    A, dt = -torch.rand(H, device="cuda", generator=g), torch.zeros(H, device="cuda")
+    outs = []
+    for spoil in (False, True):
+        x, gates = qkv.clone(), ba.clone()
+        if spoil:  # head 0
+            if what in "qkv":
+                x[row, {"q": 0, "k": H * dk, "v": 2 * H * dk}[what] + 5] = bad
+            else:
+                gates[row, 0 if what == "beta" else H] = float("nan") if what == "beta" else bad
+        state = torch.zeros((H, dk, dv), device="cuda")
+        outs.append((ops.delta_rule_chunked(x, gates, A, dt, H, dk, dv, state), state))
+    (want, s0), (got, s1) = outs
+    assert torch.equal(got[:row], want[:row])
+    assert torch.equal(got[:, dv:], want[:, dv:]) and torch.equal(s1[1], s0[1])
+    assert not torch.isfinite(got[row, :dv]).all()
+
+
 @pytest.mark.parametrize("M,H,dv", [(1, 16, 128), (9, 3, 80), (4, 2, 256), (2, 5, 7)])
 def test_delta_norm_matches_oracle(hip, M, H, dv):
     from webgllm_amd import ops

@@ -16,6 +16,8 @@
 // once a launch, whatever the row count. Per row, two barriers that wait on
 // LDS only: one after q, k and the gates are in LDS, one after the partial
 // S^T k^ and S^T q^ are; the next row's inputs load across them.
+#include <type_traits>
+
 #include "common.h"
 #include "epilogue.h"
 
@@ -323,7 +325,7 @@ constexpr int RS = CMAX + 4;  // LDS row stride (floats) of the row tiles: rows 
 constexpr int AS = CH + 4;    // LDS row stride of A and P
 constexpr int TS = 20;        // LDS row stride of the inverted diagonal blocks
 constexpr int CW = 8;         // waves a workgroup
-constexpr size_t PREP_LDS = (2 * CH * RS + 2 * CH * AS + CH * TS + 4 * CH) * sizeof(float);
+constexpr size_t PREP_LDS = (2 * CH * RS + 2 * CH * AS + CH * TS + 4 * CH + 4) * sizeof(float);
 typedef float f4v __attribute__((ext_vector_type(4)));
 
 struct ChunkArgs {
@@ -355,6 +357,32 @@ __device__ __forceinline__ f4v mma16(f4v a, f4v b, f4v c) {
   return c;
 }
 
+// (16 x 16 lower triangular m) b. CAREFUL: a value of b that is not finite
+// is kept from the rows before its own, which m's zeros there times it would
+// make NaN: those rows come from b without such values.
+template <bool CAREFUL>
+__device__ __forceinline__ f4v mma16_lower(f4v m, f4v b) {
+  const f4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f4v r = mma16(m, b, zero);
+  if constexpr (CAREFUL) {
+    const int row = 4 * ((threadIdx.x & 63) >> 4);
+    int first = 16;  // this column's first row that is not finite
+#pragma unroll
+    for (int e = 3; e >= 0; e--)
+      if (!isfinite(b[e])) {
+        b[e] = 0.0f;
+        first = row + e;
+      }
+    first = min(first, __shfl_xor(first, 16, 64));
+    first = min(first, __shfl_xor(first, 32, 64));
+    const f4v f = mma16(m, b, zero);
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (row + e < first) r[e] = f[e];
+  }
+  return r;
+}
+
 // Bound by MFMA: 1920 of them (15,360 clocks over 4 SIMDs) a workgroup. As
 // vector code (one wave a SIMD, T by a serial forward substitution of 64
 // rows) 1500 rows of 16 heads took 141 us; this takes 46 us.
@@ -364,6 +392,7 @@ __global__ __launch_bounds__(64 * CW) void delta_chunk_prep_kernel(ChunkArgs a) 
   float *sA = sk + CH * RS, *sP = sA + CH * AS;  // -A and P
   float *sT = sP + CH * AS;                      // (I + A_ii)^-1 of the diagonal blocks
   float *sG = sT + CH * TS, *sB = sG + CH, *sE = sB + CH, *sL = sE + CH;  // G, beta, e^G, e^(Gl-G)
+  float *sF = sL + CH;  // whether a gate or key is not finite
   const int c = blockIdx.x, h = blockIdx.y, t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int ln = lane & 15, lg = lane >> 4;
@@ -372,7 +401,8 @@ __global__ __launch_bounds__(64 * CW) void delta_chunk_prep_kernel(ChunkArgs a) 
   const int K = a.H * a.dk, dk = a.dk, dv = a.dv;
   const int KT = (dk + 15) / 16, VT = (dv + 15) / 16;
   // every load issued before the first store: thread t takes column t % 128
-  // of rows 4 u + t / 128; a wave its 16 value columns
+  // of rows 4 u + t / 128; a wave its 16 value columns (rows and columns past
+  // the chunk read its last, without a branch, and become 0)
   f4v x[CT];  // this wave's value columns: rows 16 i + 4 lg + e, column 16 wave + ln
   {
     const int i = t & (CMAX - 1), r0 = t >> 7;
@@ -380,10 +410,9 @@ __global__ __launch_bounds__(64 * CW) void delta_chunk_prep_kernel(ChunkArgs a) 
 #pragma unroll
     for (int u = 0; u < CH / 4; u++) {
       const int r = 4 * u + r0;
-      const float *row = a.qkv + (int64_t)(c0 + r) * a.ldq;
-      const bool in = r < n && i < dk;
-      rq[u] = in ? row[h * dk + i] : 0.0f;
-      rk[u] = in ? row[K + h * dk + i] : 0.0f;
+      const float *row = a.qkv + (int64_t)(c0 + min(r, n - 1)) * a.ldq;
+      rq[u] = row[h * dk + min(i, dk - 1)];
+      rk[u] = row[K + h * dk + min(i, dk - 1)];
     }
     const int vj = 16 * wave + ln;
 #pragma unroll
@@ -391,13 +420,19 @@ __global__ __launch_bounds__(64 * CW) void delta_chunk_prep_kernel(ChunkArgs a) 
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const int r = 16 * i2 + 4 * lg + e;
-        x[i2][e] = r < n && vj < dv ? a.qkv[(int64_t)(c0 + r) * a.ldq + 2 * K + h * dv + vj] : 0.0f;
+        x[i2][e] = a.qkv[(int64_t)(c0 + min(r, n - 1)) * a.ldq + 2 * K + h * dv + min(vj, dv - 1)];
       }
 #pragma unroll
     for (int u = 0; u < CH / 4; u++) {
-      sq[(4 * u + r0) * RS + i] = rq[u];
-      sk[(4 * u + r0) * RS + i] = rk[u];
+      const bool in = 4 * u + r0 < n && i < dk;
+      sq[(4 * u + r0) * RS + i] = in ? rq[u] : 0.0f;
+      sk[(4 * u + r0) * RS + i] = in ? rk[u] : 0.0f;
     }
+#pragma unroll
+    for (int i2 = 0; i2 < CT; i2++)
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (16 * i2 + 4 * lg + e >= n || vj >= dv) x[i2][e] = 0.0f;
   }
   if (t < CH) {  // wave 0: the gates (LIN_GATES) and G by a shuffle scan (linCum)
     float beta = 0.0f, g = 0.0f;
@@ -412,12 +447,16 @@ __global__ __launch_bounds__(64 * CW) void delta_chunk_prep_kernel(ChunkArgs a) 
       const float y = __shfl_up(g, off, 64);
       if (lane >= off) g += y;
     }
-    const float gl = __shfl(g, n - 1, 64);
+    const float gl = __shfl(g, n - 1, 64), eg = expf(g);
+    const bool bad = __ballot(!isfinite(beta) || !isfinite(g) || !isfinite(eg)) != 0;
     sB[t] = beta;
     sG[t] = g;
-    sE[t] = expf(g);
+    sE[t] = eg;
     sL[t] = expf(gl - g);
-    if (t == 0) a.eg[h * a.nch + c] = expf(gl);
+    if (t == 0) {
+      a.eg[h * a.nch + c] = expf(gl);
+      *sF = bad ? 1.0f : 0.0f;
+    }
   }
   lds_barrier();
   {  // LIN_PREP: eight threads a row
@@ -434,6 +473,7 @@ __global__ __launch_bounds__(64 * CW) void delta_chunk_prep_kernel(ChunkArgs a) 
     }
     const float invq = 1.0f / sqrtf((float)dk) / sqrtf(ssq + 1e-6f);
     const float invk = 1.0f / sqrtf(ssk + 1e-6f);
+    if (part == 0 && !isfinite(ssk)) *sF = 1.0f;
     for (int i = part; i < dk; i += 8) {
       sq[r * RS + i] *= invq;
       sk[r * RS + i] *= invk;
@@ -495,44 +535,64 @@ __global__ __launch_bounds__(64 * CW) void delta_chunk_prep_kernel(ChunkArgs a) 
   }
   lds_barrier();
   // linUW by blocks: X_i = T_ii (R_i - sum_j<i A_ij X_j), this wave's value
-  // columns (R = beta V) and key columns (R = beta e^G K^).
+  // columns (R = beta V) and key columns (R = beta e^G K^); then linQO: Oi =
+  // P U, Q' = e^G Q^ + P (-W).
   const f4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
-  f4v y[CT], qp[CT];
+  f4v y[CT], qp[CT], o[CT], off = zero;
+  auto solve = [&](auto careful) {
+    constexpr bool CAREFUL = decltype(careful)::value;
 #pragma unroll
-  for (int i = 0; i < CT; i++)
+    for (int i = 0; i < CT; i++)
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int r = 16 * i + 4 * lg + e;
-      const float b = sB[r], ex = sE[r];
-      x[i][e] *= b;
-      y[i][e] = sk[r * RS + 16 * wave + ln] * (b * ex);
-      qp[i][e] = sq[r * RS + 16 * wave + ln] * ex;
+      for (int e = 0; e < 4; e++) {
+        const int r = 16 * i + 4 * lg + e;
+        const float b = sB[r], ex = sE[r];
+        x[i][e] *= b;
+        y[i][e] = sk[r * RS + 16 * wave + ln] * (b * ex);
+        qp[i][e] = sq[r * RS + 16 * wave + ln] * ex;
+        if constexpr (!CAREFUL) off[e] = fmaf(x[i][e], 0.0f, off[e]);
+      }
+#pragma unroll
+    for (int i = 0; i < CT; i++) {
+#pragma unroll
+      for (int j = 0; j < i; j++) {  // (each block's sum by itself, then added)
+        const f4v m = *reinterpret_cast<const f4v *>(sA + (16 * i + ln) * AS + 16 * j + 4 * lg);
+        x[i] += mma16(m, x[j], zero);
+        y[i] += mma16(m, y[j], zero);
+      }
+      const f4v m = *reinterpret_cast<const f4v *>(sT + (16 * i + ln) * TS + 4 * lg);
+      x[i] = mma16_lower<CAREFUL>(m, x[i]);
+      y[i] = mma16_lower<CAREFUL>(m, y[i]);
     }
 #pragma unroll
-  for (int i = 0; i < CT; i++) {
+    for (int i = 0; i < CT; i++) y[i] = -y[i];
 #pragma unroll
-    for (int j = 0; j < i; j++) {  // (each block's sum by itself, then added)
-      const f4v m = *reinterpret_cast<const f4v *>(sA + (16 * i + ln) * AS + 16 * j + 4 * lg);
-      x[i] += mma16(m, x[j], zero);
-      y[i] += mma16(m, y[j], zero);
+    for (int i = 0; i < CT; i++) {
+      o[i] = zero;
+#pragma unroll
+      for (int j = 0; j <= i; j++) {
+        const f4v m = *reinterpret_cast<const f4v *>(sP + (16 * i + ln) * AS + 16 * j + 4 * lg);
+        o[i] += j < i ? mma16(m, x[j], zero) : mma16_lower<CAREFUL>(m, x[j]);
+        qp[i] += j < i ? mma16(m, y[j], zero) : mma16_lower<CAREFUL>(m, y[j]);
+      }
     }
-    const f4v m = *reinterpret_cast<const f4v *>(sT + (16 * i + ln) * TS + 4 * lg);
-    x[i] = mma16(m, x[i], zero);
-    y[i] = mma16(m, y[i], zero);
-  }
+  };
+  solve(std::false_type{});
+  // Where a value (off is NaN), a key or a gate is not finite: again, with the
+  // rows before it kept from it.
+  if (__builtin_expect(__ballot((off[0] + off[1]) + (off[2] + off[3]) + *sF != 0.0f) != 0, 0)) {
+    // (none of the first loads' addresses and masks kept for these)
+    const float *v = a.qkv + (int64_t)c0 * a.ldq + 2 * K + h * dv + 16 * wave + ln;
+    int rows = 16 * wave + ln < dv ? n : 0;
+    asm volatile("" : "+v"(v), "+v"(rows));
 #pragma unroll
-  for (int i = 0; i < CT; i++) y[i] = -y[i];
-  // linQO: Oi = P U, Q' = e^G Q^ + P (-W)
-  f4v o[CT];
+    for (int i = 0; i < CT; i++)
 #pragma unroll
-  for (int i = 0; i < CT; i++) {
-    o[i] = zero;
-#pragma unroll
-    for (int j = 0; j <= i; j++) {
-      const f4v m = *reinterpret_cast<const f4v *>(sP + (16 * i + ln) * AS + 16 * j + 4 * lg);
-      o[i] += mma16(m, x[j], zero);
-      qp[i] += mma16(m, y[j], zero);
-    }
+      for (int e = 0; e < 4; e++) {
+        const int r = 16 * i + 4 * lg + e;
+        x[i][e] = r < rows ? v[(int64_t)r * a.ldq] : 0.0f;
+      }
+    solve(std::true_type{});
   }
   if (wave < VT) {
 #pragma unroll
