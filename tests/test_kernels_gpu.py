@@ -437,6 +437,35 @@ def test_attn_prefill_wave_splits(hip, waves, H, KV, hd, M, pos0):
         assert rel_l2(got[m], want) <= 1e-3, m
 
 
+@pytest.mark.parametrize("waves", [1, 2, 3])
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("bad", [32, 40, 63, 95])
+def test_attn_prefill_keeps_earlier_rows(hip, waves, hd, bad):
+    """A cached value row that is not finite: every row that does not see it
+    has a clean cache's output (run again in another order of sums: the
+    parity bar); the rows that see it come out as no number (the largest
+    half, as a NaN is stored)."""
+    from webgllm_amd import lib as L, ops
+    H, M = 2, 96  # (one query head a KV head: a wave is 32 rows)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(bad)
+    q = torch.randn((M, H * hd), device="cuda", generator=g) / hd ** 0.5
+    k, v = (torch.randn((M, H * hd), device="cuda", generator=g).half() for _ in range(2))
+    pos = torch.zeros(1, dtype=torch.int32, device="cuda")
+    shape = ops.attn_shape(H, H, hd, hd, 1e-6, False)
+    old = L.tuning_get("attn_prefill_mfma")
+    L.tuning_set("attn_prefill_mfma", waves)
+    try:
+        want = ops.attn_prefill(q, shape, k, v, pos)
+        v[bad] = float("nan")
+        got = ops.attn_prefill(q, shape, k, v, pos)
+    finally:
+        L.tuning_set("attn_prefill_mfma", old)
+    for m in range(bad):
+        assert rel_l2(got[m].float().cpu().numpy(), want[m].float().cpu().numpy()) <= 1e-3, m
+    assert (got[bad:].abs() == 65504).all()
+
+
 @pytest.mark.parametrize("M,D,W", [(1, 2048, 3), (5, 2048, 3), (8, 1024, 4), (40, 512, 3)])
 def test_short_conv_and_accept(hip, M, D, W):
     from webgllm_amd import ops

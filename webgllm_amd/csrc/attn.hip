@@ -1925,6 +1925,39 @@ void attn_prefill_mfma_kernel(
       m_run = mx;
     }
   }
+  // A key that a query does not see has a weight of 0, but 0 times a value
+  // that is not finite is NaN. Where a sum is not finite the wave's queries
+  // run again, a lane each over the keys it sees (half the dims a lane).
+  float nan = 0.0f;
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+    for (int j = 0; j < 16; j++) nan = fmaf(o[dt][j], 0.0f, nan);
+  if (__builtin_expect(qvalid && nan != 0.0f, 0)) {
+    const float *qp = q + (int64_t)qm * ldq + (int64_t)(kh * G + qs % G) * HD;
+    m_run = -INFINITY;
+    l_run = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+      for (int j = 0; j < 16; j++) o[dt][j] = 0.0f;
+    for (int key = 0; key <= q_last; key++) {
+      const _Float16 *kp = reinterpret_cast<const _Float16 *>(k_cache) + (int64_t)key * kvd + kh * HD;
+      const _Float16 *vp = reinterpret_cast<const _Float16 *>(v_cache) + (int64_t)key * kvd + kh * HD;
+      float s = 0.0f;
+#pragma unroll 8
+      for (int d = 0; d < HD; d++) s = fmaf(qp[d], (float)kp[d], s);
+      const float m_new = fmaxf(m_run, s), mu = m_new == -INFINITY ? 0.0f : m_new;
+      const float corr = __expf(m_run - mu), w = __expf(s - mu);
+      l_run = l_run * corr + w;
+      m_run = m_new;
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+        for (int j = 0; j < 16; j++)
+          o[dt][j] = fmaf(w, (float)vp[32 * dt + 8 * (j >> 2) + 4 * hh + (j & 3)], o[dt][j] * corr);
+    }
+  }
   if (qvalid) {
     const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
     uint16_t *op = out + (int64_t)qm * ldo + (int64_t)(kh * G + qs % G) * HD;
