@@ -466,6 +466,36 @@ def test_attn_prefill_keeps_earlier_rows(hip, waves, hd, bad):
     assert (got[bad:].abs() == 65504).all()
 
 
+@pytest.mark.parametrize("waves", [1, 2, 3])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_attn_prefill_queries_near_the_largest_half(hip, waves, hd):
+    """Queries of up to 65504, which times log2 e are past the largest half:
+    the rows' outputs against float64, as any other row's."""
+    from webgllm_amd import lib as L, ops
+    H, M = 2, 40
+    rng = np.random.default_rng(hd)
+    q = rng.standard_normal((M, H * hd)).astype(np.float32) / 8
+    k, v = (rng.standard_normal((M, H * hd)).astype(np.float16) for _ in range(2))
+    q[::3, 5] = 65504
+    q[1::3, hd + 7] = -50000
+    k[:, [5, hd + 7]] *= np.float16(1e-4)
+    shape = ops.attn_shape(H, H, hd, hd, 1e-6, False)
+    old = L.tuning_get("attn_prefill_mfma")
+    L.tuning_set("attn_prefill_mfma", waves)
+    try:
+        got = ops.attn_prefill(_t(q), shape, _t(k), _t(v), _t(np.zeros(1, np.int32)))
+    finally:
+        L.tuning_set("attn_prefill_mfma", old)
+    got = got.cpu().numpy().astype(np.float64)
+    for m in range(M):
+        for h in range(H):
+            c = slice(h * hd, h * hd + hd)
+            s = k[:m + 1, c].astype(np.float64) @ q[m, c].astype(np.float64)
+            w = np.exp(s - s.max())
+            want = w @ v[:m + 1, c].astype(np.float64) / w.sum()
+            assert rel_l2(got[m, c], want) <= 1e-3, (m, h)
+
+
 @pytest.mark.parametrize("M,D,W", [(1, 2048, 3), (5, 2048, 3), (8, 1024, 4), (40, 512, 3)])
 def test_short_conv_and_accept(hip, M, D, W):
     from webgllm_amd import ops

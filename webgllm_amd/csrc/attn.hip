@@ -1926,8 +1926,9 @@ void attn_prefill_mfma_kernel(
     }
   }
   // A key that a query does not see has a weight of 0, but 0 times a value
-  // that is not finite is NaN. Where a sum is not finite the wave's queries
-  // run again, a lane each over the keys it sees (half the dims a lane).
+  // that is not finite is NaN; and a query past 45,400 is past the largest
+  // half once it is times log2 e. Queries whose sums are not finite run again,
+  // a lane each over the keys it sees (half the dims a lane).
   float nan = 0.0f;
 #pragma unroll
   for (int dt = 0; dt < DT; dt++)
