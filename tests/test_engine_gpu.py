@@ -411,24 +411,59 @@ def test_verify_grows_the_cache(hip, family):
     assert kept2 == kept and tokens == written
 
 
+def _prompt_rows_in_turn(eng, M):
+    """A prompt batch's layers as one operation after another, what
+    wg_prefill_layers issues."""
+    from webgllm_amd import ops
+    s, b = eng.shape, eng._pre_buffers()
+    h, x16, rs = b["h"][:M], b["x16"][:M], b["rs"][:M]
+    ops.embed(eng.w.embedding, b["ids"][:M], out=h)
+    for i, lw in enumerate(eng.w.layers):
+        ops.norm_to_h2(h, lw["op_norm"], s.eps, x16, rs)
+        if s.layer_type(i) == "conv":
+            bcx = ops.gemm(lw["in_proj"], x16, out=b["bcx"][:M], row_scale=rs)
+            ops.short_conv(bcx, s.hidden, s.conv_kernel, lw["taps"], eng.state[i],
+                           out=b["c16"][:M])
+            ops.gemm(lw["out_proj"], b["c16"][:M], out=h, residual=h)
+        else:
+            qkv = ops.gemm(lw["qkv"], x16, out=b["qkv"][:M], col_of=eng._col_of(lw["qkv"]),
+                           row_scale=rs)
+            ops.head_prep(qkv, eng.attn, eng.rope, eng.pos, eng.k_cache[i], eng.v_cache[i],
+                          lw.get("q_norm"), lw.get("k_norm"), q_out=b["q"][:M])
+            ops.attn_prefill(b["q"][:M], eng.attn, eng.k_cache[i], eng.v_cache[i], eng.pos,
+                             out=b["att16"][:M])
+            ops.gemm(lw["o"], b["att16"][:M], out=h, residual=h)
+        ops.norm_to_h2(h, lw["ffn_norm"], s.eps, x16, rs)
+        ops.gemm_swiglu(lw["gate_up"], x16, out=b["ff16"][:M], row_scale=rs)
+        ops.gemm(lw["down"], b["ff16"][:M], out=h, residual=h)
+
+
 @pytest.mark.parametrize("family", sorted(FAMILIES))
 def test_prompt_layers_in_one_call_equal_the_calls_in_turn(hip, family):
-    """A prompt's layers from the native call and, with a probe set, one
-    operation at a time: the same logits, caches and states bit for bit, on a
-    new sequence, a continued one and after the caches have grown."""
+    """A prompt's layers from one native call, from one a layer with a probe
+    between them, and one operation at a time: the same logits, caches and
+    states bit for bit, on a new sequence, a continued one and after the
+    caches have grown."""
     outs = []
-    for probe in (None, lambda *a: None):
+    for form in ("one call", "probe", "in turn"):
         eng, _ = _pair(family, seed=5, ctx=1024)
         rng = np.random.default_rng(1)
-        got = []
+        got, seen = [], []
+        if form == "in turn":
+            eng._prefill_rows = lambda M, eng=eng: _prompt_rows_in_turn(eng, M)
         for n in (9, 40, 300):
-            eng.probe = probe
+            if form == "probe":
+                eng.probe = lambda i, name, rows: seen.append((i, name))
             picks = eng.forward(_prompt(rng, n, eng.shape.vocab))
             eng.probe = None
             got += [picks, eng.logits[:len(picks)].clone()]
+        if form == "probe" and eng._prefill_ok():
+            attn = [i for i in range(eng.shape.layers) if eng.shape.layer_type(i) == "attn"]
+            assert seen == [(i, "attention") for _ in range(3) for i in attn]
         for i in sorted(eng.k_cache):
             got += [eng.k_cache[i][:eng.position], eng.v_cache[i][:eng.position]]
         outs.append(got + [eng.state[i] for i in sorted(eng.state)])
     torch.cuda.synchronize()
-    for a, b in zip(*outs):
-        assert torch.equal(a, b)
+    for other in outs[1:]:
+        for a, b in zip(outs[0], other):
+            assert torch.equal(a, b)

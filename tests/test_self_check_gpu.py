@@ -55,3 +55,19 @@ def test_self_check_catches_a_wrong_attention(hip, monkeypatch):
     finally:
         for k, v in saved.items():
             L.tuning_set(k, v)
+
+
+def test_self_check_runs_the_prompt_path(hip, monkeypatch):
+    """A fault in what a prompt runs (one head of the attention's output
+    zeroed after the native layer call) is seen by the check, whose prompt
+    takes the same call."""
+    w = E.Weights(SHAPES["llama"], seed=12)
+    hd, real, engines = SHAPES["llama"].head_dim, ops.prefill_layers, []
+
+    def zero_head(layers, batch):
+        real(layers, batch)
+        engines[-1]._pre_buffers()["att16"][:, hd:2 * hd].zero_()
+
+    monkeypatch.setattr(E.ops, "prefill_layers", zero_head)
+    engines.append(E.Engine(w, 256))
+    assert S.self_check(engines[-1]) > S.SELF_CHECK_MAX

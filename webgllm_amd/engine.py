@@ -281,7 +281,8 @@ class Engine:
         self._cols = {}   # device row orders of the matrices (GEMM column maps)
         # probe(layer, name, rows), called as the forward enqueues (not under
         # graph capture): ("embedding", h rows) after the lookup, ("attention",
-        # (q rows, output rows)) after each attention, ("output", h rows)
+        # (q rows, output rows)) after each attention (a prompt batch's: after
+        # its layer), ("output", h rows)
         # after the last layer; the self-check reads them back
         self.probe = None
         # short convs in in_proj's epilogue (False: in_proj, then the conv)
@@ -547,34 +548,18 @@ class Engine:
         reference's prescaled half(h w / 32), its 32 / RMS the GEMM's row
         scale, as in the few-token path; the caches and conv states advance;
         no head here (_prefill_head). The layers run from one native call, or,
-        for a probe between them, from here."""
-        s, w, b = self.shape, self.w, self._pre_buffers()
-        D = s.hidden
-        h, x16, rs = b["h"][:M], b["x16"][:M], b["rs"][:M]
-        ops.embed(w.embedding, b["ids"][:M], out=h)
+        for a probe between them, from a call each: a layer's queries and
+        attention output stand in their buffers until the next layer's."""
+        b = self._pre_buffers()
+        ops.embed(self.w.embedding, b["ids"][:M], out=b["h"][:M])
+        layers, batch = self._prefill_layers(), self._prefill_batch(M)
         if not self.probe:
-            ops.prefill_layers(self._prefill_layers(), self._prefill_batch(M))
+            ops.prefill_layers(layers, batch)
             return
-        for i, lw in enumerate(w.layers):
-            ops.norm_to_h2(h, lw["op_norm"], s.eps, x16, rs)
-            if s.layer_type(i) == "conv":
-                bcx = ops.gemm(lw["in_proj"], x16, out=b["bcx"][:M], row_scale=rs)
-                ops.short_conv(bcx, D, s.conv_kernel, lw["taps"], self.state[i], out=b["c16"][:M])
-                ops.gemm(lw["out_proj"], b["c16"][:M], out=h, residual=h)
-            else:
-                qkv = ops.gemm(lw["qkv"], x16, out=b["qkv"][:M], col_of=self._col_of(lw["qkv"]),
-                               row_scale=rs)
-                ops.head_prep(qkv, self.attn, self.rope, self.pos, self.k_cache[i],
-                              self.v_cache[i], lw.get("q_norm"), lw.get("k_norm"),
-                              q_out=b["q"][:M])
-                ops.attn_prefill(b["q"][:M], self.attn, self.k_cache[i], self.v_cache[i],
-                                 self.pos, out=b["att16"][:M])
-                if self.probe:
-                    self.probe(i, "attention", (b["q"][:M], b["att16"][:M]))
-                ops.gemm(lw["o"], b["att16"][:M], out=h, residual=h)
-            ops.norm_to_h2(h, lw["ffn_norm"], s.eps, x16, rs)
-            ops.gemm_swiglu(lw["gate_up"], x16, out=b["ff16"][:M], row_scale=rs)
-            ops.gemm(lw["down"], b["ff16"][:M], out=h, residual=h)
+        for i, layer in enumerate(layers):
+            ops.prefill_layers((L.PrefillLayer * 1)(layer), batch)
+            if not layer.conv_width:
+                self.probe(i, "attention", (b["q"][:M], b["att16"][:M]))
 
     def _prefill_head(self, r0: int, T: int) -> None:
         """Logits and picks of rows r0 .. r0 + T - 1 (T <= 8) of the last
