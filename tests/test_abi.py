@@ -107,6 +107,18 @@ def test_repack_rejects_mismatched_layouts():
     assert "without them" in L.last_error()
 
 
+def test_records_past_32_bits_are_refused():
+    """A Q4_K-record matrix whose records (or groups of blocks) do not count
+    in 32 bits: refused, where the count had been cut to its low bits."""
+    lib = L.load()
+    N, K = (1 << 31) - 4, 1 << 20
+    m = L.Q4MatrixDesc(N, K, L.LAYOUT_ROWGROUP, L.ZERO_Q4K, 4096, 4096, None)
+    for rc in (lib.wg_repack_q4_k(C.byref(m), 0, N, 4096, None, None),
+               lib.wg_q4k_record_halves(C.byref(m), 1 << 60, 1 << 61, None)):
+        assert rc == -1  # WG_ERR_INVALID
+        assert b"past 2^32" in lib.wg_last_error()
+
+
 def test_tuning_knobs():
     assert L.tuning_get("gemv_min_waves") >= 0
     old = L.tuning_get("gemv_wg_per_cu")

@@ -179,11 +179,13 @@ def test_few_rows_take_the_kept_halves(hip, N, K):
             assert rel_l2(_np(yb), _np(ya)) <= 2e-4, M
 
 
-@pytest.mark.parametrize("N,K,offset", [(4, 256, 0), (12, 768, 4), (68, 2304, 1)])
+@pytest.mark.parametrize("N,K,offset", [(4, 256, 0), (12, 768, 4), (68, 2304, 1),
+                                        (8 * (16 * 16384 + 17), 256, 0)])
 def test_records_repack_and_halves_at_any_alignment(hip, N, K, offset):
     """Source bytes and halves buffers off their 16- and 8-byte alignment, and
-    the rows written in two ranges: the same quants and halves as the
-    half-zero-point repack of the whole."""
+    the rows written in two ranges (of the largest, one in two rows of
+    workgroups): the same quants and halves as the half-zero-point repack of
+    the whole."""
     import ctypes as C
     from webgllm_amd import lib as L, ops
     rng = np.random.default_rng(N + K + offset)

@@ -135,13 +135,12 @@ template <bool A16>
 __global__ __launch_bounds__(256) void repack_q4_k_rec_kernel(uint4 *quants, uint32_t *recs,
                                                               const uint8_t *src,
                                                               const int32_t *src_rows, int row0,
-                                                              uint32_t threads, int supers) {
-  // 32-bit thread counts: 2^32 threads would be a 155 GB matrix, which the
-  // device cannot hold beside its source (a 64-bit division cost more)
-  const uint32_t t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= threads) return;  // (threads: a multiple of 16, so whole records leave)
-  const int r = (int)(t & 3), pair = (int)(t >> 2) & 3;
-  const uint32_t gs = t >> 4;
+                                                              uint32_t records, int supers) {
+  // 16 records a workgroup; 32-bit record numbers (a 64-bit division cost
+  // more), which the caller bounds
+  const uint32_t gs = (blockIdx.y * gridDim.x + blockIdx.x) * 16 + (threadIdx.x >> 4);
+  if (gs >= records) return;  // (whole records leave)
+  const int r = (int)(threadIdx.x & 3), pair = (int)(threadIdx.x >> 2) & 3;
   const int gi = (int)(gs / (uint32_t)supers), s = (int)(gs % (uint32_t)supers);
   const int i = 4 * gi + r;
   const uint8_t *p = src + ((int64_t)(src_rows ? src_rows[i] : i) * supers + s) * 144;
@@ -496,6 +495,8 @@ inline unsigned grid_for(int64_t threads, int per) { return (unsigned)((threads 
 int launch_q4k_expand(const wg_q4_matrix *w, uint16_t *scales, uint16_t *zeros, hipStream_t s) {
   const int blocks = w->K / 32;
   const int64_t n = (int64_t)(w->N / 4) * blocks;
+  WG_REQUIRE(n <= 0xffffffffll - 256,
+             "Q4_K record expansion: a %d x %d matrix is past 2^32 groups of blocks", w->N, w->K);
   const bool wide = ((uintptr_t)w->scales & 15) == 0 &&
                     (((uintptr_t)scales | (uintptr_t)zeros) & 7) == 0;
   auto kernel = wide ? q4k_rec_expand_kernel<true> : q4k_rec_expand_kernel<false>;
@@ -567,12 +568,18 @@ int wg_repack_q4_k(const wg_q4_matrix *m, int32_t row0, int32_t rows, const void
   if (m->zero == WG_ZERO_Q4K) {
     WG_REQUIRE(row0 % 4 == 0 && rows % 4 == 0,
                "wg_repack_q4_k: rows must start and end on a row group");
-    const int64_t n = (int64_t)(rows / 4) * supers * 16;
+    // Even rows of up to 16,384 workgroups: a grid dimension holds under 2^32
+    // threads.
+    const int64_t records = (int64_t)(rows / 4) * supers, blocks = (records + 15) / 16;
+    WG_REQUIRE(records <= 0xffffffffll - (16 << 16),
+               "wg_repack_q4_k: %d rows of %d are past 2^32 records", rows, m->K);
+    const int64_t gy = (blocks + 16383) / 16384;
+    const dim3 grid((unsigned)((blocks + gy - 1) / gy), (unsigned)gy);
     auto kernel = ((uintptr_t)src & 15) == 0 ? repack_q4_k_rec_kernel<true>
                                              : repack_q4_k_rec_kernel<false>;
-    kernel<<<grid_for(n, 256), 256, 0, as_stream(stream)>>>(
-        (uint4 *)m->quants, (uint32_t *)m->scales, (const uint8_t *)src, src_rows, row0,
-        (uint32_t)n, supers);
+    kernel<<<grid, 256, 0, as_stream(stream)>>>((uint4 *)m->quants, (uint32_t *)m->scales,
+                                                (const uint8_t *)src, src_rows, row0,
+                                                (uint32_t)records, supers);
     return launched("wg_repack_q4_k");
   }
   int64_t n = (int64_t)rows * supers * 4;
