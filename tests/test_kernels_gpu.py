@@ -334,9 +334,10 @@ def _prefill_case(H, KV, hd, M, pos0, seed, ctx=None, nan_past=False):
     return q, k, v, _h(out)
 
 
-@pytest.fixture(params=[4, 1, 0], ids=["mfma4", "mfma1", "valu"])
+@pytest.fixture(params=[3, 4, 1, 0], ids=["mfma", "mfma4", "mfma1", "valu"])
 def prefill_kernel(request):
-    """wg_attn_prefill's kernel: MFMA with 4 or 1 waves a workgroup, or VALU."""
+    """wg_attn_prefill's kernel: MFMA as the shape chooses, with 4 or 1 waves of
+    queries a workgroup, or VALU."""
     from webgllm_amd import lib as L
     old = L.tuning_get("attn_prefill_mfma")
     L.tuning_set("attn_prefill_mfma", request.param)
@@ -417,7 +418,7 @@ def test_head_prep_of_prompt_rows(hip, H, KV, hd, norm, pos0):
             assert torch.equal(x, y)
 
 
-@pytest.mark.parametrize("waves", [1, 2, 3])
+@pytest.mark.parametrize("waves", [1, 2, 4])
 @pytest.mark.parametrize("H,KV,hd", [(14, 2, 64), (32, 8, 128), (64, 2, 64)])
 @pytest.mark.parametrize("M,pos0", [(1, 0), (9, 22), (17, 47), (33, 63), (70, 190)])
 def test_attn_prefill_wave_splits(hip, waves, H, KV, hd, M, pos0):
@@ -437,7 +438,7 @@ def test_attn_prefill_wave_splits(hip, waves, H, KV, hd, M, pos0):
         assert rel_l2(got[m], want) <= 1e-3, m
 
 
-@pytest.mark.parametrize("waves", [1, 2, 3])
+@pytest.mark.parametrize("waves", [1, 2, 4])
 @pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("bad", [32, 40, 63, 95])
 def test_attn_prefill_keeps_earlier_rows(hip, waves, hd, bad):
@@ -466,7 +467,7 @@ def test_attn_prefill_keeps_earlier_rows(hip, waves, hd, bad):
     assert (got[bad:].abs() == 65504).all()
 
 
-@pytest.mark.parametrize("waves", [1, 2, 3])
+@pytest.mark.parametrize("waves", [1, 2, 4])
 @pytest.mark.parametrize("hd", [64, 128])
 def test_attn_prefill_queries_near_the_largest_half(hip, waves, hd):
     """Queries of up to 65504, which times log2 e are past the largest half:

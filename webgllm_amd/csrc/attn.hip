@@ -2210,8 +2210,8 @@ int wg_attn_prefill(const float *q, int32_t M, int32_t ldq, const wg_attn_shape 
     // 6000, past the line, 135 against 126); from four a compute unit at 128
     // dims, four of queries (2048 rows over 8192 keys 475 against 508, the
     // tiles read by half as many groups; 90 against 85 from position 0).
-    const bool few = form == 4 ? pairs < cus : form == 1;
-    const bool wide = hd == 128 && (form == 4 ? pairs >= 4 * (int64_t)cus : form == 3);
+    const bool few = form == 3 ? pairs < cus : form == 1;
+    const bool wide = hd == 128 && (form == 3 ? pairs >= 4 * (int64_t)cus : form == 4);
 #define WG_PF_LAUNCH(HD, QW, KW, KT)                                                        \
   launch_prefill_mfma<HD, QW, KW, KT>(q, M, ldq, H, KV, k_cache, v_cache, pos0, max_keys, out, \
                                       ldo, s)

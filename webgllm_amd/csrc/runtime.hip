@@ -86,7 +86,7 @@ static Knob g_knobs[] = {
     {"gemv_mfma", 1, 0, 2},              // row-group GEMV on MFMA: 1 for 3 to 8 tokens, 2 also 1 and 2, 0 never
     {"gemv_mfma_wg_per_cu", 0, 0, 16},   // its persistent workgroups per CU (0: by shape)
     {"gemv_mfma_pairs", 4, 2, 8},        // its block pairs a wave (2, 4, 8)
-    {"attn_prefill_mfma", 4, 0, 4},      // prompt attention on MFMA: 4 chooses; 1, 2, 3: 1, 2 or 4 waves of queries a workgroup (4, 2, 1 of keys; 3 at 128 dims), 0 VALU
+    {"attn_prefill_mfma", 3, 0, 4},      // prompt attention on MFMA: waves of queries a workgroup (1, 2, 4; 4 is 2 at 64 dims), the others of keys; 3 chooses, 0 VALU
     {"attn_mfma", 1, 0, 2},              // decode attention in one launch on MFMA: 1 where it is faster (past 8 queries a KV head, from 16384 keys, outside the XCD-grouped split form's range with KV heads a multiple of 8, else up to 2048 keys), 2 always, 0 never
     {"attn_fused", 1, 0, 2},             // decode attention in one launch: 1 where it is faster, 2 always, 0 never
     {"attn_xcd", 1, 0, 2},               // decode attention with each XCD combining its own KV heads (a multiple of 8): 1 the split form up to 4 queries a KV head below 4096 keys and the MFMA form grouped, 2 the split form always, 0 never
