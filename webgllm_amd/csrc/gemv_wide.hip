@@ -128,7 +128,7 @@ struct Q8 {
 };
 
 struct Q6K {
-  static int per_cu(int G) { return G >= 24576 ? 4 : 2; }
+  static int per_cu(int G) { return G >= 26624 ? 4 : 2; }
   static constexpr int AV = 8;
   static constexpr int NSUM = 4;
   template <int NB>
@@ -366,10 +366,14 @@ int launch_stream(const Mat &mat, int G, const uint16_t *x, int ldx, float *y, i
                   const wg_epilogue &e, hipStream_t s) {
   constexpr int RGW = 4 / KS;
   // Workgroups a compute unit: the knob, or 2, and more for a vocabulary's
-  // row groups, whose many rounds a slow workgroup would hold up (us at 2 /
-  // 4 / 8, one row: Q6_K 128256 x 4096 83.2 / 79.1 / 80.3, 65536 x 2048 31.3 /
-  // 32.4 / 34.0, 20000 x 4096 18.5 / 19.8 / 21.8; 8-bit 128256 x 4096 99.1 /
-  // 95.0 / 93.3, 65536 x 2048 28.6 / 27.6 / 27.4, 16384 x 2048 9.8 at each).
+  // row groups, whose many rounds a slow workgroup would hold up. One row, us
+  // in a graph at 2 / 4 / 8, by row groups of 4: Q6_K 2048 deep 20,480 38.8 /
+  // 39.5 / 40.7, 24,576 45.5 / 46.3 / 47.3, 26,624 48.6 / 48.4 / 50.5, 32,064
+  // 58.4 / 56.5 / 59.3; 4096 deep 12,288 36.2 / 36.2 / 39.4, 24,576 65.4 /
+  // 65.6 / 68.0, 26,624 70.9 / 69.8 / 71.7, 32,064 84.1 / 81.5 / 83.8. 8-bit
+  // 1024 deep 12,288 14.8 / 13.9 / 14.9, 16,384 18.9 / 17.2 / 17.4; 4096 deep
+  // 14,336 46.6 / 44.9 / 46.2, 16,384 53.4 / 52.0 / 52.5, 24,576 77.3 / 76.8 /
+  // 75.9, 37,984 116.3 / 116.4 / 116.1.
   int per_cu = tuning("wide_wg_per_cu");
   if (!per_cu) per_cu = M == 1 ? F::per_cu(G) : 2;  // (two rows: equal or slower)
   int grid = persistent_grid((G + RGW - 1) / RGW, per_cu);
