@@ -1662,10 +1662,12 @@ __device__ inline half2v split_rest(half2v hi, float a, float b) {
 // one step ahead. KW wave groups of QW waves: a group's waves share its
 // tiles, and the groups take the key steps in turn (KW > 1 where the
 // queries alone leave compute units idle), their sums merged in LDS.
-// Bound by the matrix cores (twice the products for the hi / lo splits) and
-// by the vector work a key and query. 2048 rows over 8192 keys, 32 heads
-// over 8 of 128: 1020 us with single-buffered tiles, 2-byte value reads and
-// a mask and rescale every 32 keys; 440 now (1.09 PFLOP/s of products).
+// Bound by neither pipe alone but by a wave's own chain of scores, softmax and
+// values, which two waves a SIMD cover in part: 2048 rows over 8192 keys, 32
+// heads over 8 of 128, run the matrix cores 42% of the time (twice the
+// products for the hi / lo splits) and the vector units 31%. 1020 us with
+// single-buffered tiles, 2-byte value reads and a mask and rescale every 32
+// keys; 420 to 440 now, by the box, in a graph (1.1 PFLOP/s of products).
 // K and V rows past the block's last visible key (or the cache) are loaded
 // from the step's first row instead: stale bits never reach an MFMA.
 template <int HD, int QW, int KW, int KT>
@@ -2205,11 +2207,15 @@ int wg_attn_prefill(const float *q, int32_t M, int32_t ldq, const wg_attn_shape 
     const int G = H / KV, cus = persistent_grid(1 << 30, 1);
     const int64_t pairs = (int64_t)KV * ((M + 64 / G - 1) / (64 / G));  // of waves of 32 queries
     // Two waves of queries and two of keys; where those workgroups are fewer
-    // than the compute units, one of queries and four of keys (8B heads: 256
-    // rows at 1000 20 us against 28, 45 at 6000 59 against 102; 512 rows at
-    // 6000, past the line, 135 against 126); from four a compute unit at 128
-    // dims, four of queries (2048 rows over 8192 keys 475 against 508, the
-    // tiles read by half as many groups; 90 against 85 from position 0).
+    // than the compute units, one of queries and four of keys. Kernel alone in
+    // a graph, us, four of keys / two, 32 heads over 8: 45 rows at 6000 58 /
+    // 103, 256 at 1000 20 / 28, 256 at 0 10.4 / 11.8; past the line 512 at 6000
+    // 128 / 117, 512 at 0 19.8 / 16.5; just before it (12 heads over 2) 1024
+    // at 0 22.9 / 24.5, at 6000 127 / 123. From four a compute unit at 128
+    // dims, four of queries, whose tiles half as many groups read (none of
+    // keys / two: 2048 rows at 6144 419 / 430, at 14336 853 / 892, but at 2048
+    // 200 / 195 and at 0 87 / 83; three a compute unit, 1536 at 0, 61 / 55; two,
+    // 1024 at 6000, 217 / 206).
     const bool few = form == 3 ? pairs < cus : form == 1;
     const bool wide = hd == 128 && (form == 3 ? pairs >= 4 * (int64_t)cus : form == 4);
 #define WG_PF_LAUNCH(HD, QW, KW, KT)                                                        \

@@ -383,9 +383,11 @@ __device__ __forceinline__ f4v mma16_lower(f4v m, f4v b) {
   return r;
 }
 
-// Bound by MFMA: 1920 of them (15,360 clocks over 4 SIMDs) a workgroup. As
-// vector code (one wave a SIMD, T by a serial forward substitution of 64
-// rows) 1500 rows of 16 heads took 141 us; this takes 46 us.
+// Bound by its phases in turn (loads, norms, products, solve, products), which
+// the one workgroup that 108 KB of LDS leave a compute unit does not overlap:
+// its 1920 MFMA are 6.4 us of the SIMDs, and 1500 rows of 16 heads (384
+// workgroups, two rounds) take 46 us, MFMA busy 21%. As vector code (one wave
+// a SIMD, T by a serial forward substitution of 64 rows) they took 141 us.
 __global__ __launch_bounds__(64 * CW) void delta_chunk_prep_kernel(ChunkArgs a) {
   extern __shared__ __align__(16) float sm[];
   float *sq = sm, *sk = sq + CH * RS;            // q^, k^ rows (0 past n, dims); then Q', -W
@@ -632,10 +634,11 @@ struct ChainIn {
 
 // A workgroup per (head, 16 state columns): waves 0 to 3 a row tile of D
 // each, 4 to 7 one of O, then every wave its 16 state rows. The state and D
-// pass between the waves through LDS as fragments. Bound by MFMA (384 a
-// chunk, 3072 clocks over 4 SIMDs) and the two exchanges a chunk. The
-// fragments come one chunk ahead. As vector code over LDS tiles a chunk took
-// 7.6 us, 1500 rows 184 us; this takes 66 us.
+// pass between the waves through LDS as fragments; the memory's come one
+// chunk ahead. Bound by the chain of a chunk: 384 MFMA (1.3 us of 4 SIMDs) and
+// two exchanges in 2.8 us, on one compute unit in two at 16 heads of 128 (MFMA
+// busy 23% of them all, 46% of those in use). As vector code over LDS tiles a
+// chunk took 7.6 us, 1500 rows 184 us; this takes 66 us.
 __global__ __launch_bounds__(64 * CW) void delta_chunk_chain_kernel(ChunkArgs a) {
   __shared__ __align__(16) float sS[2][KTM][256], sD[CT][256];
   // blockIdx.x is the head: the workgroups of one head (consecutive in

@@ -11,7 +11,7 @@
 //    weights in flight under the third, and no wave waits for another until
 //    the end;
 //  - one MFMA is one 32-weight block of 16 columns, its weights q - z exact
-//    halves, so the block's scale multiplies its exact float32 sum;
+//    halves: exact products, whose float32 sum the block's scale multiplies;
 //  - the waves' sums meet in LDS once, in the waves' order.
 // An operand: lane (n = lane % 16, c = lane / 16) holds activations 8 c ..
 // 8 c + 7 of the block's 32 in row n, and the same 8 weights of column n:
