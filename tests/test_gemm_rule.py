@@ -22,9 +22,9 @@ def rule(tmp_path_factory):
     d = tmp_path_factory.mktemp("rule")
     src, so = d / "rule.cpp", d / "rule.so"
     src.write_text(f'#include "{CSRC}/gemm_rule.h"\n'
-                   'extern "C" int tile(int zk, int M, int N, int K, int cus, int groups,'
-                   ' int splits) {\n'
-                   '  return wg::gemm_tile_for(zk, M, N, K, cus, groups != 0, splits != 0);\n}\n')
+                   'extern "C" int tile(int zk, int M, int N, int K, int cus, int residual,'
+                   ' int groups, int splits) {\n'
+                   '  return wg::gemm_tile_for(zk, M, N, K, cus, residual, groups, splits);\n}\n')
     subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-o",
                     str(so), str(src)], check=True)
     return C.CDLL(str(so))
@@ -36,8 +36,8 @@ def test_plain_settings_take_no_wave_groups(rule):
     assert PLAIN_TUNING["gemm_splits"] == 1
     for zk in ZK.values():
         for M, N, K in SIZES:
-            assert rule.tile(zk, M, N, K, CUS, 0, 0) <= 3, (zk, M, N, K)
-    assert any(rule.tile(0, M, N, K, CUS, 1, 1) >= 4 for M, N, K in SIZES)
+            assert max(rule.tile(zk, M, N, K, CUS, r, 0, 0) for r in (0, 1)) <= 3, (zk, M, N, K)
+    assert any(rule.tile(0, M, N, K, CUS, 0, 1, 1) >= 4 for M, N, K in SIZES)
 
 
 # (form, M, N, K, the tile where splits may run, the tile under capture): each
@@ -60,8 +60,22 @@ def test_plain_settings_take_no_wave_groups(rule):
     ("f16", 300, 9728, 8448, 2, 2), ("q4_0", 300, 4096, 14336, 1, 1), ("q8", 257, 6144, 8448, 1, 1),
     ("f16", 300, 1152, 14336, 1, 1), ("q4_0", 400, 1152, 8448, 1, 1)])
 def test_lines(rule, zk, M, N, K, tile, captured):
-    assert rule.tile(ZK[zk], M, N, K, CUS, 1, 1) == tile
-    assert rule.tile(ZK[zk], M, N, K, CUS, 1, 0) == captured
+    assert rule.tile(ZK[zk], M, N, K, CUS, 0, 1, 1) == tile
+    assert rule.tile(ZK[zk], M, N, K, CUS, 0, 1, 0) == captured
+
+
+# (form, M, N, K, the tile where a residual is added, without one)
+@pytest.mark.parametrize("zk,M,N,K,tile,plain", [
+    ("q4_0", 700, 1024, 4608, 7, 5), ("q4_0", 400, 2048, 8192, 7, 5), ("q8", 700, 1024, 4608, 5, 5),
+    ("f16", 300, 2048, 6144, 7, 5), ("f16", 300, 2048, 7168, 5, 5), ("u8", 300, 2048, 7168, 7, 1),
+    ("u8", 300, 2048, 8192, 1, 1), ("q4_0", 100, 9728, 4096, 4, 1), ("q4_0", 1024, 1152, 5632, 4, 1),
+    ("f16", 1500, 896, 8192, 4, 2), ("q8", 1024, 1152, 8192, 4, 2), ("f16", 2048, 2048, 2048, 1, 2),
+    ("u8", 64, 8704, 7168, 1, 1), ("q4_0", 64, 8704, 4096, 5, 5), ("q4_0", 65, 8192, 4096, 7, 5),
+    ("q8", 65, 9216, 2048, 4, 7), ("q8", 65, 9216, 2560, 7, 7), ("q8", 400, 4096, 8448, 1, 2),
+    ("q8", 400, 5120, 8448, 2, 2), ("u8", 300, 4096, 14336, 1, 2), ("f16", 400, 4096, 8448, 2, 2)])
+def test_lines_of_a_residual(rule, zk, M, N, K, tile, plain):
+    assert rule.tile(ZK[zk], M, N, K, CUS, 1, 1, 1) == tile
+    assert rule.tile(ZK[zk], M, N, K, CUS, 0, 1, 1) == plain
 
 
 def test_tiles_divide_the_columns(rule):
@@ -69,5 +83,5 @@ def test_tiles_divide_the_columns(rule):
     cols = {0: 64, 1: 128, 2: 128, 3: 256, 4: 128, 5: 64, 6: 32, 7: 64, 8: 128}
     for zk in ZK.values():
         for M, N, K in SIZES + [(M, N + 64, K) for M, N, K in SIZES]:
-            for groups, splits in ((1, 1), (1, 0), (0, 0)):
-                assert N % cols[rule.tile(zk, M, N, K, CUS, groups, splits)] == 0
+            for form in ((0, 1, 1), (1, 1, 1), (0, 1, 0), (1, 1, 0), (0, 0, 0)):
+                assert N % cols[rule.tile(zk, M, N, K, CUS, *form)] == 0

@@ -770,8 +770,8 @@ int launch(const wg_q4_matrix *w, const uint16_t *A, int M, int lda, float *C, i
   if (t == 0) {
     const int cus = persistent_grid(1 << 30, 1);
     const bool groups = tuning("gemm_splits") == 0;
-    t = gemm_tile_for(ZK, M, w->N, w->K, cus, groups, groups);
-    const int whole = gemm_tile_for(ZK, M, w->N, w->K, cus, groups, false);
+    t = gemm_tile_for(ZK, M, w->N, w->K, cus, residual, groups, groups);
+    const int whole = gemm_tile_for(ZK, M, w->N, w->K, cus, residual, groups, false);
     if (t != whole && capturing(s)) t = whole;
   }
 #define WG_GROUPS(BM, BN, S, WN, KG) \
