@@ -1664,10 +1664,11 @@ __device__ inline half2v split_rest(half2v hi, float a, float b) {
 // queries alone leave compute units idle), their sums merged in LDS.
 // Bound by neither pipe alone but by a wave's own chain of scores, softmax and
 // values, which two waves a SIMD cover in part: 2048 rows over 8192 keys, 32
-// heads over 8 of 128, run the matrix cores 42% of the time (twice the
-// products for the hi / lo splits) and the vector units 31%. 1020 us with
-// single-buffered tiles, 2-byte value reads and a mask and rescale every 32
-// keys; 420 to 440 now, by the box, in a graph (1.1 PFLOP/s of products).
+// heads over 8 of 128, run the matrix cores 42% of the time at 2.4 GHz, 54% of
+// the clocks that they leave the chip (twice the products for the hi / lo
+// splits), and the vector units 31%. 1020 us with single-buffered tiles, 2-byte
+// value reads and a mask and rescale every 32 keys; 420 to 440 now, by the box,
+// in a graph (1.1 PFLOP/s of products).
 // K and V rows past the block's last visible key (or the cache) are loaded
 // from the step's first row instead: stale bits never reach an MFMA.
 template <int HD, int QW, int KW, int KT>
